@@ -1581,7 +1581,7 @@ void pack_udt(Executor* x, std::vector<UdtItem>& items, int apply_pivot) {
   std::vector<UdtItem> tab;
   for (int p = 0; p < np; p++) {
     tab.clear();
-    for (int R : {1, 2, 4, 8})
+    for (int R : {1, 8})
       for (size_t i = 0; i < items.size(); i++) {
         if (p >= (int)st[i].size()) continue;
         UdtItem u = items[i];

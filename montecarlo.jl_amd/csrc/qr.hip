@@ -8,8 +8,8 @@
 // and T = D^-1 R, column-permuted (apply_pivot) or left "dirty upper" for rdivp.
 //
 // GPU form (a short sequence of launches per batch of matrices):
-//  * Blocked Householder with panels of w <= 16 columns factorised in LDS by one
-//    workgroup, and the trailing matrix updated with the compact-WY block reflector
+//  * Blocked Householder with panels of w <= 16 columns factorised by one workgroup (one
+//    wave per column), and the trailing matrix updated with the compact-WY block reflector
 //    I - V T V^T by one wave per 16-column strip on the matrix cores, so the trailing
 //    matrix is streamed once per panel instead of once per column.  The same launch
 //    accumulates Q = H_1 ... H_P forward on 16-row strips of U (U <- U (I - V T V^T),
@@ -29,9 +29,7 @@
 
 namespace dqmc {
 
-constexpr int kQrThreads = 256;
 constexpr int kQrMaxW = 16;
-constexpr int kPanelDoubles = 4 * 64 * 17;  // the column steps' reduction transposes
 
 // Wave64 sum of a double, result in every lane: butterflies inside each 16-lane row
 // with DPP (quad_perm xor 1, xor 2, row_ror 4, row_ror 8), then the four row sums are
@@ -69,19 +67,11 @@ __device__ __forceinline__ dx4 mfma16(double a, double b, dx4 c) {
 // between launches: it.tau holds the residual norms, it.pivot the working permutation,
 // it.tfac the taus of each panel.
 
-// Rows of the panel per thread of the panel kernel (256 threads): 1, 2, 4 or 8.
-
-__host__ __device__ static int udt_rows_per_thread(int rows) {
-  int R = 1;
-  while (R * 256 < rows) R *= 2;
-  return R;
-}
-
-// Panel width for `rows` remaining rows: the panel lives in registers (R rows x w columns
-// per thread, at most 64 values).
+// Panel width for `rows` remaining rows: one wave per column, the panel's reflectors held in
+// LDS (width x rows doubles, at most 128 KB), so 16 columns up to 1024 rows and 8 beyond.
+constexpr int kPanelWideRows = 1024;
 __host__ __device__ static int udt_panel_width(int rows) {
-  int w = 64 / udt_rows_per_thread(rows);
-  if (w > kQrMaxW) w = kQrMaxW;
+  int w = rows <= kPanelWideRows ? kQrMaxW : kQrMaxW / 2;
   if (w > rows) w = rows;
   if (w < 1) w = 1;
   return w;
@@ -181,437 +171,323 @@ __device__ __forceinline__ void bitonic64(double& kv, int& ki, int lane) {
   bitonic_stage<64, 32>(kv, ki, lane);
 }
 
-static size_t udt_panel_lds_bytes(int n) {
-  size_t b = 0;
-  b += (size_t)n * 8;                 // nrm
-  b += (size_t)kPanelDoubles * 8;     // the factorisation's reduction transposes
-  b += 32 * 8;                        // taus, scalars
-  b += 2 * (4 * 16 + 16) * 8;         // wave totals, row j (two buffers)
-  b += 4 * 16 * 16;                   // top-16 candidates of each wave
-  b += (size_t)n * 4;                 // perm
-  b += 3 * 32 * 4 + 16;               // moves, selection, misc
-  return b;
+// Sum of a double over the wave, wave-uniform: butterflies inside each 16-lane row, then the
+// row totals through row_bcast 15 (rows 1 and 3 take the row below) and row_bcast 31 (rows 2
+// and 3 take lane 31), so lane 63 holds the total.
+__device__ __forceinline__ double wave_total(double v) {
+  v += dpp_mov<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_mov<0x124>(v);  // row_ror 4
+  v += dpp_mov<0x128>(v);  // row_ror 8
+  {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x142, 0xA, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x142, 0xA, 0xF, false);
+    v += __hiloint2double(hi, lo);
+  }
+  {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x143, 0xC, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x143, 0xC, 0xF, false);
+    v += __hiloint2double(hi, lo);
+  }
+  return readlane_d(v, 63);
 }
 
-// Column steps J.. of the single-wave panel factorisation (rows <= 256: lane l holds rows
-// l + 64 k; rows at or beyond `rows` hold zeros, so they add nothing and stay zero).  A
-// template recursion, so every register index is a compile-time constant, and branch-free
-// inside a step: only row block k = 0 holds rows <= j, selected per lane.
-// Per step: the partial sums of ||x||^2 and x^T a_c (c > j) are transposed through LDS
-// (lane 4 v + g adds value v of 16 lanes, quads combined with DPP) together with row j,
-// so lane 4 c holds column c's sum and a_jc and computes its w_c; the w_c reach every
-// lane by readlane.
-template <int J, int RT, int WM>
-__device__ __forceinline__ void panel_steps_wave(double (&a)[RT][WM], double (&taus)[WM], double* rw, int lane,
-                                                 int w) {
-  if constexpr (J < WM) {
-    constexpr int j = J;
-    taus[j] = 0.0;
-    if (j < w) {
-      double* rj = rw + 64 * 17;          // row j of the panel
-      double part[WM];
-      {
-        const double x0 = a[0][j];
-        const double xe = lane >= j ? x0 : 0.0;
-        const double xg = lane > j ? x0 : 0.0;
-        part[j] = xe * xe;
-#pragma unroll
-        for (int c = j + 1; c < WM; c++) part[c] = xg * a[0][c];
-      }
-#pragma unroll
-      for (int k = 1; k < RT; k++) {
-        const double x = a[k][j];
-        part[j] += x * x;
-#pragma unroll
-        for (int c = j + 1; c < WM; c++) part[c] += x * a[k][c];
-      }
-#pragma unroll
-      for (int c = j; c < WM; c++) rw[lane * 17 + c] = part[c];
-      if (lane == j) {
-#pragma unroll
-        for (int c = j; c < WM; c++) rj[c] = a[0][c];
-      }
-      __builtin_amdgcn_wave_barrier();
-      const int v = lane >> 2, g = lane & 3;
-      double s4[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 0; q < 16; q++) s4[q & 3] += rw[(g * 16 + q) * 17 + v];
-      const double ajv = rj[v];
-      double sv = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-      __builtin_amdgcn_wave_barrier();
-      sv += dpp_mov<0xB1>(sv);             // quad_perm [1,0,3,2]
-      sv += dpp_mov<0x4E>(sv);             // quad_perm [2,3,0,1]
-      const double normu = readlane_d(sv, 4 * j);
-      const double xi1 = readlane_d(ajv, 4 * j);
-      if (normu != 0.0) {                  // wave-uniform
-        const double nu = copysign(sqrt(normu), xi1);
-        const double xi = xi1 + nu;
-        const double tau = xi / nu;
-        const double rxi = 1.0 / xi;
-        const double wl = tau * (ajv + sv * rxi);   // w_v in lanes 4 v .. 4 v + 3
-        double wc[WM];
-#pragma unroll
-        for (int c = j + 1; c < WM; c++) wc[c] = readlane_d(wl, 4 * c);
-        {
-          const double x0 = a[0][j];
-          const double vv = x0 * rxi;
-          const double coef = lane > j ? vv : (lane == j ? 1.0 : 0.0);
-          a[0][j] = lane > j ? vv : (lane == j ? -nu : x0);
-#pragma unroll
-          for (int c = j + 1; c < WM; c++) a[0][c] -= coef * wc[c];
-        }
-#pragma unroll
-        for (int k = 1; k < RT; k++) {
-          const double vv = a[k][j] * rxi;
-          a[k][j] = vv;
-#pragma unroll
-          for (int c = j + 1; c < WM; c++) a[k][c] -= vv * wc[c];
-        }
-        taus[j] = tau;
-      }
-    }
-    panel_steps_wave<J + 1, RT, WM>(a, taus, rw, lane, w);
+// nu = copysign(||x||, x1), xi = x1 + nu and g = 1 / (nu xi) from normu = ||x||^2 > 0, so that
+// H a = a - u (u^T a) g with u = (xi, x_2, x_3, ...).  Inside a range where nothing can overflow
+// or turn subnormal the root comes from the hardware estimate by Goldschmidt's iteration and the
+// reciprocal by Newton's (each refined past double precision); outside, the library forms.
+__device__ __forceinline__ void reflector_scalars(double normu, double x1, double& nu, double& xi, double& g) {
+  if (normu >= 0x1p-900 && normu <= 0x1p900) {
+    const double y = __builtin_amdgcn_rsq(normu);
+    double s = normu * y, h = 0.5 * y;
+    const double r = fma(-s, h, 0.5);
+    s = fma(s, r, s);
+    h = fma(h, r, h);
+    s = fma(fma(-s, s, normu), h, s);
+    s = fma(fma(-s, s, normu), h, s);
+    nu = copysign(s, x1);
+    xi = x1 + nu;
+    const double den = fma(fabs(x1), s, normu);    // nu xi
+    double q = __builtin_amdgcn_rcp(den);
+    q = fma(fma(-den, q, 1.0), q, q);
+    q = fma(fma(-den, q, 1.0), q, q);
+    g = q;
+  } else {
+    nu = copysign(sqrt(normu), x1);
+    xi = x1 + nu;
+    g = 1.0 / (nu * xi);
   }
 }
 
-// Column steps J.. of the four-wave panel factorisation (thread t holds rows t + 256 k).
-// A template recursion, so every register index is a compile-time constant.  The row-j
-// and total buffers alternate with the step parity, so one barrier per step suffices.
-template <int J, int R, int WM>
-__device__ __forceinline__ void panel_steps_block(double (&a)[R][WM], double* red, double* wt, double* rowj,
-                                                  double* sc, int tid, int lane, int wave, int rows, int w) {
-  if constexpr (J < WM) {
-    constexpr int j = J;
-    if (j < w) {
-    const int bsel = j & 1;
-    double* wtb = wt + bsel * 64;
-    double* rjb = rowj + bsel * 16;
-    double part[WM];
+// LDS of a panel workgroup of NWV waves and RT rows per lane: the published columns (the pivot
+// choice's candidate lists alias them), the steps' scalars, the progress counters, the choice.
+template <int RT, int NWV>
+constexpr size_t panel_lds() { return (size_t)NWV * 64 * RT * 8 + 32 * 8 + 4 * 4 + 16 * 4; }
+
+// The w largest residual norms of columns [p0, n) in order, ties to the lower column
+// (reference: strict ">"), into selr.  Every 64 columns are sorted by one wave, which keeps
+// their best 16; groups of four such lists are merged until one is left.  With the odd lists of
+// a group stored reversed, the 64 candidates are in the state the bitonic network reaches after
+// its size-16 stage, so a merge is its size-32 and size-64 stages.  A NaN norm orders as the
+// largest and is counted as a device error.
+template <int RT, int NWV>
+__device__ __forceinline__ void panel_choice(const UdtItem& it, int n, int p0, int w, int lane, int wave, double* cv,
+                                             int* selr) {
+  constexpr int kLists = RT < 4 ? 4 : RT;            // RT lists, padded to whole groups of four
+  constexpr int kMerged = kLists <= 4 ? 0 : kLists <= 16 ? 4 : 8 + 4;   // lists of the later levels
+  static_assert((kLists + kMerged) * 16 * 12 <= NWV * 64 * RT * 8, "lists fit the columns they alias");
+  int* ci = reinterpret_cast<int*>(cv + (kLists + kMerged) * 16);
+  for (int l = wave; l < kLists; l += NWV) {
+    const int k = p0 + 64 * l + lane;
+    double kv = k < n ? it.tau[k] : -HUGE_VAL;
+    int ki = k;
+    const bool bad = kv != kv;
+    if (bad) kv = HUGE_VAL;
+    if (__ballot(bad) && lane == 0 && it.err) atomicAdd(it.err, 1ull);
+    if (p0 + 64 * l < n) bitonic64(kv, ki, lane);    // (an empty list is in order)
+    if (RT == 1) {
+      if (l == 0 && lane < 16) selr[lane] = lane < w ? ki : p0;
+    } else if (lane < 16) {
+      const int slot = l * 16 + ((l & 1) ? 15 - lane : lane);
+      cv[slot] = kv;
+      ci[slot] = ki;
+    }
+  }
+  __syncthreads();
+  if constexpr (RT > 1) {
+    int base = 0;
 #pragma unroll
-    for (int c = 0; c < WM; c++) part[c] = 0.0;
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const int i = tid + 256 * k;
-      if (i < rows && i >= j) {
-        const double x = a[k][j];
-        part[j] += x * x;
-        if (i > j) {
-#pragma unroll
-          for (int c = j + 1; c < WM; c++) part[c] += x * a[k][c];
+    for (int lists = kLists; lists > 1;) {
+      const int groups = lists / 4, pad = groups > 1 ? (groups + 3) / 4 * 4 : 1;
+      for (int m = wave; m < pad; m += NWV) {
+        double kv = -HUGE_VAL;
+        int ki = n + 4096 + m * 64 + lane;
+        if (m < groups) {
+          kv = cv[base + m * 64 + lane];
+          ki = ci[base + m * 64 + lane];
+          bitonic_stage<32, 16>(kv, ki, lane);
+          bitonic_stage<64, 32>(kv, ki, lane);
+        }
+        if (pad == 1) {
+          if (lane < 16) selr[lane] = lane < w ? ki : p0;
+        } else if (lane < 16) {
+          const int slot = base + lists * 16 + m * 16 + ((m & 1) ? 15 - lane : lane);
+          cv[slot] = kv;
+          ci[slot] = ki;
         }
       }
-      if (i == j) {
-#pragma unroll
-        for (int c = 0; c < WM; c++) rjb[c] = a[k][c];
-      }
+      __syncthreads();
+      base += lists * 16;
+      lists = pad;
     }
-    double* rw = red + (size_t)(wave * 64) * 17;
-#pragma unroll
-    for (int c = 0; c < WM; c++) rw[lane * 17 + c] = part[c];
-    __builtin_amdgcn_wave_barrier();
-    {
-      constexpr int GL = 64 / WM;            // lanes per value after the transpose
-      const int v = lane / GL, g = lane % GL;
-      double s4[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 0; q < WM; q++) s4[q & 3] += rw[(g * WM + q) * 17 + v];
-      double sv = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-      sv += dpp_mov<0xB1>(sv);             // quad_perm [1,0,3,2]
-      sv += dpp_mov<0x4E>(sv);             // quad_perm [2,3,0,1]
-      if (GL == 8) sv += dpp_mov<0x141>(sv);   // row_half_mirror: the other quad of 8
-      if (g == 0) wtb[wave * 16 + v] = sv;
-    }
-    __syncthreads();
-    double tot;
-    {
-      const int v = lane % WM;
-      tot = (wtb[v] + wtb[16 + v]) + (wtb[32 + v] + wtb[48 + v]);
-    }
-    const double normu = readlane_d(tot, j);
-    const double xi1 = rjb[j];
-    double tau = 0.0, nu = 0.0, xi = 1.0;
-    if (normu != 0.0) {
-      nu = copysign(sqrt(normu), xi1);
-      xi = xi1 + nu;
-      tau = xi / nu;
-    }
-    const double rxi = 1.0 / xi;
-    double wc[WM];
-#pragma unroll
-    for (int c = 0; c < WM; c++) wc[c] = c > j ? tau * (rjb[c] + readlane_d(tot, c) * rxi) : 0.0;
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const int i = tid + 256 * k;
-      if (normu != 0.0 && i < rows) {
-        if (i > j) {
-          const double vv = a[k][j] * rxi;
-          a[k][j] = vv;
-#pragma unroll
-          for (int c = j + 1; c < WM; c++) a[k][c] -= vv * wc[c];
-        } else if (i == j) {
-          a[k][j] = -nu;
-#pragma unroll
-          for (int c = j + 1; c < WM; c++) a[k][c] -= wc[c];
-        }
-      }
-    }
-    if (tid == 0) sc[j] = tau;
-    }
-    panel_steps_block<J + 1, R, WM>(a, red, wt, rowj, sc, tid, lane, wave, rows, w);
   }
 }
 
-// Householder panel of one item: pivot choice for the panel, column moves, factorisation
-// with the panel rows in registers (R rows x WM columns per thread), the taus.
-// Per column step one block reduction gives ||x||^2 and x^T a_c for the later columns:
-// with v = (x + nu e_j) / (x_j + nu), v^T a_c = a_jc + (x_{>j}^T a_c{>j}) / (x_j + nu).
-template <int R, int WM, bool TAB>
-__global__ __launch_bounds__(kQrThreads) void udt_panel_kernel(UdtBatch batch, int p0a, int wa, int lasta) {
-  constexpr bool tab = TAB;
-  const UdtItem it = tab ? batch.items[blockIdx.x] : batch.it[blockIdx.x];
-  const int n = tab ? it.n : batch.n;
-  const int p0 = tab ? it.p0 : p0a, w = tab ? it.w : wa, last = tab ? it.last : lasta;
+// Householder panel of one item: pivot choice, column moves, factorisation, the taus.
+//
+// One wave per panel column (lane l holds rows l + 64 k, k < RT), so a column step is a few
+// instructions per wave and the waves' work runs beside each other.  Column j, once final, is
+// published in LDS (x below its diagonal, zero elsewhere); every later column's wave forms its
+// x^T a while column j's wave forms ||x||^2 and the scalars, and then applies
+//   a <- a - u (u^T a) g,  u = (xi, x), g = 1 / (nu xi)   (reflector_scalars).
+// A column's wave depends only on lower columns' waves of the same workgroup, in order, so the
+// waits end; the chain is 16 steps of one reduction, one root and one reciprocal.
+// What bounds it is that chain's latency, and beside it the issue slots of the 16 waves on four
+// SIMDs.  Against one wave for all columns (up to 256 rows) and four waves with a barrier per step
+// and an n^2 count for the choice (above), per launch, one or two matrices:
+//   1024 rows 183 -> 21 us, 512 rows 77 -> 16 us, 256 rows 19.8 -> 14.0 us, 64 rows 19 -> 12.5 us;
+// a sweep of 32x32 sites 382 -> 230 ms, 24x24 323 -> 215 ms, 16x16 72.6 -> 66.8 ms.
+//
+// The swaps of the reference ("slot p0 + t <-> slot that holds choice t", t = 0, 1, ...) leave
+// choice t in slot p0 + t.  A panel column that was not chosen ends in the slot of a choice from
+// outside the panel: the path choice t -> the choice that was column p0 + t -> ... ends at it,
+// since every swap stays among the slots and columns of one such path.  Waves 0 to 3, done with
+// their columns first, move the columns; a row is moved by one lane, which reads all its sources
+// before it writes.
+template <int RT, int NWV>
+__device__ __forceinline__ void panel_body(const UdtItem& it, int n, int p0, int w, int last, unsigned char* smem) {
+  constexpr int LR = 64 * RT;
   const int rows = n - p0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  extern __shared__ __align__(16) unsigned char smem[];
-  double* nrm = reinterpret_cast<double*>(smem);
-  double* P = nrm + n;
-  double* sc = P + kPanelDoubles;   // sc[0..15] taus of the panel
-  double* red = P;               // [4][64][17] reduction transposes
-  double* wt = sc + 32;          // [2][4][16] wave totals, by step parity
-  double* rowj = wt + 2 * 64;    // [2][16] row j, by step parity
-  double* candv = rowj + 32;     // [64] top-16 norms of each wave
-  int* candi = reinterpret_cast<int*>(candv + 64);   // [64] their columns
-  int* perm = candi + 64;
-  int* mv_dst = perm + n;
-  int* mv_src = mv_dst + 32;
-  int* selr = mv_src + 32;       // 16
-  int* misc = selr + 32;         // [0] moves
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  double* V = reinterpret_cast<double*>(smem);   // [NWV][LR] published columns
+  double* scal = V + NWV * LR;                   // [16][2] xi, g of each step
+  int* pub = reinterpret_cast<int*>(scal + 32);  // [0] columns published, [1] steps' scalars published
+  int* selr = pub + 4;                           // [16] the choice
   double* __restrict__ A = it.A;
 
-  for (int k = p0 + tid; k < n; k += kQrThreads) {
-    nrm[k] = it.tau[k];
-    perm[k] = it.pivot[k];
-  }
-  if (tid < kQrMaxW) selr[tid] = -1;
-  __syncthreads();
+  if (tid < 2) pub[tid] = 0;
+  panel_choice<RT, NWV>(it, n, p0, w, lane, wave, V, selr);
 
-  // the w largest residual norms, ties to the lower index (reference: strict ">"); wave 0
-  // lane t < w ends with the t-th choice in selk
-  int selk = p0;
-  if (rows <= kQrThreads) {
-    // bitonic sort of (norm, column) best-first inside each wave; the waves' top 16 are
-    // merged in wave 0, which keeps the result in registers.  With the odd waves' lists
-    // stored reversed, the 64 candidates are in the state the bitonic network reaches after
-    // its size-16 stage (runs alternately best-first and reversed), so only the size-32 and
-    // size-64 merges remain.
-    const int k = p0 + tid;
-    double kv = k < n ? nrm[k] : -HUGE_VAL;
-    int ki = k < n ? k : n + tid;
-    bitonic64(kv, ki, lane);
-    if (lane < 16) {
-      const int slot = wave * 16 + ((wave & 1) ? 15 - lane : lane);
-      candv[slot] = kv;
-      candi[slot] = ki;
+  const int c = wave;
+  double a[RT];
+  if (c < w) {
+    const double* src = A + (size_t)p0 + (size_t)selr[c] * n;
+#pragma unroll
+    for (int k = 0; k < RT; k++) {
+      const int i = lane + 64 * k;
+      a[k] = src[i < rows ? i : rows - 1];
     }
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RT; k++) a[k] = lane + 64 * k < rows ? a[k] : 0.0;
+  }
+  // movers: lane e < w: choice e and, if it comes from outside the panel, the column that
+  // takes its slot
+  constexpr int kMovers = 4;
+  int sel = p0, out = -1;
+  if (wave < kMovers) {
+    const int le = lane & 15;
+    sel = le < w ? selr[le] : p0 + le;
+    int nxt = le;                                // the choice that was column p0 + le (else le)
+#pragma unroll
+    for (int t = 0; t < kQrMaxW; t++) nxt = __builtin_amdgcn_readlane(sel, t) == p0 + le ? t : nxt;
+#pragma unroll
+    for (int q = 0; q < 4; q++) nxt = __shfl(nxt, nxt, 64);
+    if (le < w && sel >= p0 + w) out = p0 + nxt;
     if (wave == 0) {
-      kv = candv[lane];
-      ki = candi[lane];
-      bitonic_stage<32, 16>(kv, ki, lane);
-      bitonic_stage<64, 32>(kv, ki, lane);
-      selk = ki;
-    }
-  } else {
-    for (int k = p0 + tid; k < n; k += kQrThreads) {
-      const double v = nrm[k];
-      int cnt = 0;
-      for (int k0 = p0; k0 < n; k0 += 16) {
-        double u[16];
-#pragma unroll
-        for (int q = 0; q < 16; q++) u[q] = nrm[k0 + q < n ? k0 + q : n - 1];
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int k2 = k0 + q;
-          cnt += k2 < n && ((u[q] > v) || (u[q] == v && k2 < k));
-        }
+      // the permutation: every entry is read before one is written
+      const int pv0 = it.pivot[sel < n ? sel : n - 1];
+      const int pv1 = out >= 0 ? it.pivot[out] : 0;
+      if (lane < w) {
+        it.pivot[p0 + lane] = pv0;
+        if (out >= 0) it.pivot[sel] = pv1;
       }
-      if (cnt < w) selr[cnt] = k;
     }
-    __syncthreads();
-    if (wave == 0) selk = lane < w ? selr[lane] : p0;
   }
+  __syncthreads();   // the panel's sources are read (and the candidate lists free)
 
-  // Sequential swaps "slot p0+t <-> slot holding the t-th choice" simulated by wave 0 on
-  // the at most 2w slots involved: lane q < w is slot p0+q, lane w+q the slot of choice q
-  // when that lies outside the panel.  cont = original column now held by the lane's slot.
-  if (wave == 0) {
-    const int selv = lane < w ? selk : p0;
-    const bool ok = __ballot(lane < w && !(selv >= p0 && selv < n)) == 0ull;
-    const int selc = ok ? selv : p0 + lane;                    // lane t: t-th choice
-    // (all lanes take part in the shuffle; only then is the result selected)
-    const int cw = __shfl(selc, (lane + 64 - w) & 63, 64);
-    int slot = -1;
-    if (lane < w) slot = p0 + lane;
-    else if (lane < 2 * w) slot = cw >= p0 + w ? cw : -1;
-    int cont = slot;
-    int broken = 0;
-    auto swap_step = [&](int t) {
-      const int c = __builtin_amdgcn_readlane(selc, t);
-      const unsigned long long hold = __ballot(slot >= 0 && cont == c);
-      // every choice is held by exactly one tracked slot; an empty ballot means a broken
-      // selection: the swap is skipped and the event counted as a device error
-      broken += hold ? 0 : 1;
-      const int src = hold ? __ffsll((long long)hold) - 1 : t;  // lane whose slot holds c
-      const int a_cont = __builtin_amdgcn_readlane(cont, t);      // content of slot p0+t
-      const int b_cont = __builtin_amdgcn_readlane(cont, src);
-      if (lane == t) cont = b_cont;
-      if (lane == src && src != t) cont = a_cont;
-    };
-    if (w == kQrMaxW) {       // full panels: straight-line steps
+  double nu = 0.0, tau = 0.0, xi = 0.0, normu = 0.0;
+  if (c < w) {
+    for (int j = 0; j < c; j++) {
+      if (j == c - 1) __builtin_amdgcn_s_setprio(3);   // the next column to be published
+      while (__hip_atomic_load(pub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= j) {}
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      double x[RT];
 #pragma unroll
-      for (int t = 0; t < kQrMaxW; t++) swap_step(t);
-    } else {
-      for (int t = 0; t < w; t++) swap_step(t);
+      for (int k = 0; k < RT; k++) x[k] = V[j * LR + lane + 64 * k];
+      double s0 = x[0] * a[0], s1 = 0.0;
+#pragma unroll
+      for (int k = 1; k < RT; k++) {
+        if (k & 1) s1 = fma(x[k], a[k], s1);
+        else s0 = fma(x[k], a[k], s0);
+      }
+      const double tot = wave_total(s0 + s1);
+      const double aj = readlane_d(a[0], j);
+      while (__hip_atomic_load(pub + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= j) {}
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      const double xj = scal[2 * j], g = scal[2 * j + 1];
+      if (g != 0.0) {                            // 0: a zero column, H = I
+        const double f = fma(aj, xj, tot) * g;
+        a[0] = fma(-(lane == j ? xj : x[0]), f, a[0]);
+#pragma unroll
+        for (int k = 1; k < RT; k++) a[k] = fma(-x[k], f, a[k]);
+      }
     }
-    if (broken && lane == 0 && it.err) atomicAdd(it.err, (unsigned long long)broken);
-    const bool moved = slot >= 0 && cont != slot;
-    const unsigned long long mm = __ballot(moved);
-    const int idx = __popcll(mm & ((1ull << lane) - 1ull));
-    if (moved) {
-      mv_dst[idx] = slot;
-      mv_src[idx] = cont;
+    // column c is final: x below the diagonal, then the scalars
+    const double xc = lane > c ? a[0] : 0.0;
+    if (c + 1 < w) {
+      V[c * LR + lane] = xc;
+#pragma unroll
+      for (int k = 1; k < RT; k++) V[c * LR + lane + 64 * k] = a[k];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      if (lane == 0) __hip_atomic_store(pub, c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    if (lane == 0) misc[0] = __popcll(mm);
-    // panel column q (lane q < w) comes from original column cont
-    if (lane < w) selr[lane] = cont;
+    double s0 = lane >= c ? a[0] * a[0] : 0.0, s1 = 0.0;
+#pragma unroll
+    for (int k = 1; k < RT; k++) {
+      if (k & 1) s1 = fma(a[k], a[k], s1);
+      else s0 = fma(a[k], a[k], s0);
+    }
+    normu = wave_total(s0 + s1);
+    double g = 0.0;
+    if (normu != 0.0) reflector_scalars(normu, readlane_d(a[0], c), nu, xi, g);
+    if (c + 1 < w) {
+      if (lane == 0) {
+        scal[2 * c] = xi;
+        scal[2 * c + 1] = g;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      if (lane == 0) __hip_atomic_store(pub + 1, c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (normu != 0.0) {
+      tau = xi / nu;
+      const double rxi = 1.0 / xi;
+      a[0] = lane > c ? a[0] * rxi : (lane == c ? -nu : a[0]);
+#pragma unroll
+      for (int k = 1; k < RT; k++) a[k] *= rxi;
+    }
   }
-  __syncthreads();
-
-  // physical column moves (whole columns) and the panel registers, both read from the
-  // source columns before anything is written
-  const int nm = misc[0];
-  // R == 1 (rows <= 256): wave 0 alone factorises, lane l holding rows l + 64 k (k < 4);
-  // otherwise all 256 threads, thread t holding rows t + 256 k (k < R)
-  constexpr int RT = R == 1 ? 4 : R;         // rows per participating thread
-  constexpr int TP = R == 1 ? 64 : 256;      // participating threads
-  // rows at or beyond `rows` are zero (the factorisation relies on it); threads beyond TP
-  // hold no rows
-  double a[RT][WM];
-  if (tid < TP) {
+  if (wave < kMovers) {
+    for (int r0 = 64 * wave; r0 < n; r0 += 64 * kMovers) {
+      const int rr = r0 + lane, rc = rr < n ? rr : n - 1;
+      double v[kQrMaxW], v2[kQrMaxW];
+      const bool above = r0 < p0;              // (uniform) rows < p0: R's part of the panel columns
+#pragma unroll
+      for (int e = 0; e < kQrMaxW; e++) {
+        const int d = __builtin_amdgcn_readlane(out, e), s = __builtin_amdgcn_readlane(sel, e);
+        v[e] = A[(size_t)rc + (size_t)(d >= 0 ? d : p0) * n];
+        if (above) v2[e] = A[(size_t)rc + (size_t)(e < w ? s : p0) * n];
+      }
+#pragma unroll
+      for (int e = 0; e < kQrMaxW; e++) {
+        const int d = __builtin_amdgcn_readlane(out, e), s = __builtin_amdgcn_readlane(sel, e);
+        if (d >= 0 && rr < n) A[(size_t)rr + (size_t)s * n] = v[e];
+        if (above && e < w && rr < p0) A[(size_t)rr + (size_t)(p0 + e) * n] = v2[e];
+      }
+    }
+  }
+  __syncthreads();   // the moves have read the panel's slots
+  if (c < w) {
+    double* dst = A + (size_t)p0 + (size_t)(p0 + c) * n;
 #pragma unroll
     for (int k = 0; k < RT; k++) {
-      const int i = tid + TP * k;
-      const int ic = i < rows ? i : rows - 1;
-#pragma unroll
-      for (int c = 0; c < WM; c++) {
-        const int src = c < w ? selr[c] : selr[0];
-        a[k][c] = A[(size_t)(p0 + ic) + (size_t)src * n];
-      }
+      const int i = lane + 64 * k;
+      if (i < rows) dst[i] = a[k];
     }
-#pragma unroll
-    for (int k = 0; k < RT; k++) {
-      const bool ok = tid + TP * k < rows;
-#pragma unroll
-      for (int c = 0; c < WM; c++) a[k][c] = ok ? a[k][c] : 0.0;
+    if (last && lane == c) {   // D = |diag R| (0 -> 1) of this panel
+      const double x = fabs(a[0]);
+      it.D[p0 + c] = x == 0.0 ? 1.0 : x;
     }
+    if (lane == 0) it.tfac[(size_t)p0 * 16 + c] = tau;
+  } else if (c < kQrMaxW) {
+    if (lane == 0) it.tfac[(size_t)p0 * 16 + c] = 0.0;
   }
-  if constexpr (R == 1) {
-  // wave 0 factorises the panel while waves 1-3 move the columns.  Every source read of
-  // the panel registers is issued before the barrier and every column store after it
-  // (the vector memory operations of one workgroup reach memory in issue order).  The
-  // moves leave out the rows >= p0 of the panel's columns, which the panel store writes.
-  // Single-wave factorisation: per column one wave reduction (partial sums and row j
-  // transposed through LDS, quads combined with DPP); no barrier.
-  if (wave == 1) {
-    int pn = 0;
-    if (lane < nm) pn = perm[mv_src[lane]];
-    __builtin_amdgcn_wave_barrier();
-    if (lane < nm) perm[mv_dst[lane]] = pn;
-  }
-  __syncthreads();
-  if (wave == 0) {
-    double taus[WM];
-    panel_steps_wave<0, RT, WM>(a, taus, red, lane, w);
-    if (lane == 0) {
-#pragma unroll
-      for (int j = 0; j < WM; j++) sc[j] = taus[j];
-    }
-  } else {
-    const int t = tid - 64;
-    for (int r0 = 0; r0 < n; r0 += kQrThreads - 64) {
-      const int rr = r0 + t;
-      const int rc = rr < n ? rr : n - 1;
-      double v[2 * kQrMaxW];
-#pragma unroll
-      for (int q = 0; q < 2 * kQrMaxW; q++) {
-        const int src = q < nm ? mv_src[q] : p0;
-        v[q] = A[(size_t)rc + (size_t)src * n];
-      }
-#pragma unroll
-      for (int q = 0; q < 2 * kQrMaxW; q++) {
-        const int dst = mv_dst[q < nm ? q : 0];
-        const int lim = dst < p0 + w ? p0 : n;
-        if (q < nm && rr < lim) A[(size_t)rr + (size_t)dst * n] = v[q];
-      }
-    }
-  }
-  __syncthreads();
-  for (int k = p0 + tid; k < n; k += kQrThreads) it.pivot[k] = perm[k];
-  } else {
-  int pnew = 0;
-  if (tid < nm) pnew = perm[mv_src[tid]];
-  for (int r0 = 0; r0 < n; r0 += kQrThreads) {
-    const int rr = r0 + tid;
-    const int rc = rr < n ? rr : n - 1;
-    double v[2 * kQrMaxW];
-#pragma unroll
-    for (int q = 0; q < 2 * kQrMaxW; q++) {
-      const int src = q < nm ? mv_src[q] : p0;
-      v[q] = A[(size_t)rc + (size_t)src * n];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 2 * kQrMaxW; q++)
-      if (q < nm && rr < n) A[(size_t)rr + (size_t)mv_dst[q] * n] = v[q];
-  }
-  if (tid < nm) perm[mv_dst[tid]] = pnew;
-  __syncthreads();
-  for (int k = p0 + tid; k < n; k += kQrThreads) it.pivot[k] = perm[k];
-  // factorisation, one block reduction per column: partial sums go through LDS within
-  // each wave (lane (v, g) adds value v of one group of lanes), the groups are combined
-  // with DPP inside quads / half rows, the four wave totals through LDS and one barrier.
-  panel_steps_block<0, R, WM>(a, red, wt, rowj, sc, tid, lane, wave, rows, w);
-  __syncthreads();
-  }
-  // panel -> A, and the panel's taus for the reflector launch, which forms S = V^T V and
-  // the compact-WY factor T from them (sc holds the taus since the factorisation's barrier)
-#pragma unroll
-  for (int k = 0; k < RT; k++) {
-    const int i = tid + TP * k;
-    if (tid < TP && i < rows) {
-#pragma unroll
-      for (int c = 0; c < WM; c++)
-        if (c < w) {
-          A[(size_t)(p0 + i) + (size_t)(p0 + c) * n] = a[k][c];
-          if (last && c == i) {   // D = |diag R| (0 -> 1) of this panel
-            const double x = fabs(a[k][c]);
-            it.D[p0 + i] = x == 0.0 ? 1.0 : x;
-          }
-        }
-    }
-  }
-  if (tid >= kQrThreads - kQrMaxW) {
-    const int j = tid - (kQrThreads - kQrMaxW);
-    it.tfac[(size_t)p0 * 16 + j] = j < w ? sc[j] : 0.0;
-  }
+  if (NWV < kQrMaxW && tid < kQrMaxW - NWV) it.tfac[(size_t)p0 * 16 + NWV + tid] = 0.0;
   if (last) {
     // D = |diag R| (0 -> 1) of the earlier panels (final since their launches)
-    for (int i = tid; i < p0; i += kQrThreads) {
+    for (int i = tid; i < p0; i += 64 * NWV) {
       const double x = fabs(A[(size_t)i + (size_t)i * n]);
       it.D[i] = x == 0.0 ? 1.0 : x;
     }
   }
+}
+
+// 16-column panels of at most 64 RT rows (one chain).
+template <int RT>
+__global__ __launch_bounds__(1024) void udt_panel_kernel(UdtBatch batch, int p0, int w, int last) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  panel_body<RT, 16>(batch.it[blockIdx.x], batch.n, p0, w, last, smem);
+}
+
+// Item table: each item's own panel, rows per lane by its own size.
+__global__ __launch_bounds__(1024) void udt_panel_tab_kernel(UdtBatch batch) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const UdtItem& it = batch.items[blockIdx.x];
+  const int n = it.n, p0 = it.p0, w = it.w, last = it.last, rows = n - p0;
+  if (rows <= 64) panel_body<1, 16>(it, n, p0, w, last, smem);
+  else if (rows <= 128) panel_body<2, 16>(it, n, p0, w, last, smem);
+  else if (rows <= 256) panel_body<4, 16>(it, n, p0, w, last, smem);
+  else if (rows <= 512) panel_body<8, 16>(it, n, p0, w, last, smem);
+  else panel_body<16, 16>(it, n, p0, w, last, smem);
+}
+
+// 8-column panels of 1025 to 2048 rows.
+template <bool TAB>
+__global__ __launch_bounds__(512) void udt_panel_tall_kernel(UdtBatch batch, int p0a, int wa, int lasta) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const UdtItem& it = TAB ? batch.items[blockIdx.x] : batch.it[blockIdx.x];
+  panel_body<32, 8>(it, TAB ? it.n : batch.n, TAB ? it.p0 : p0a, TAB ? it.w : wa, TAB ? it.last : lasta, smem);
 }
 
 // One workgroup per 16-column strip: X[p0:n, strip] -= V op(T) V^T X[p0:n, strip].
@@ -882,26 +758,22 @@ hipError_t launch_udt_norms(const UdtBatch& b, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int R, int WM>
+template <int RT>
 static void launch_panel_t(const UdtBatch& b, int p0, int w, int last, hipStream_t s) {
-  if (b.items)
-    hipLaunchKernelGGL((udt_panel_kernel<R, WM, true>), dim3(b.count), dim3(kQrThreads), udt_panel_lds_bytes(b.n),
-                       s, b, p0, w, last);
-  else
-    hipLaunchKernelGGL((udt_panel_kernel<R, WM, false>), dim3(b.count), dim3(kQrThreads), udt_panel_lds_bytes(b.n),
-                       s, b, p0, w, last);
+  hipLaunchKernelGGL(udt_panel_kernel<RT>, dim3(b.count), dim3(1024), (panel_lds<RT, 16>()), s, b, p0, w, last);
 }
 
 hipError_t launch_udt_panel(const UdtBatch& b, int p0, int w, int last, hipStream_t s) {
   const int rows = b.n - p0;
-  const int R = udt_rows_per_thread(rows);
-  if (w < 1 || w > udt_panel_width(rows)) return hipErrorInvalidValue;
-  switch (R) {
-    case 1: launch_panel_t<1, 16>(b, p0, w, last, s); break;
-    case 2: launch_panel_t<2, 16>(b, p0, w, last, s); break;
-    case 4: launch_panel_t<4, 16>(b, p0, w, last, s); break;
-    default: launch_panel_t<8, 8>(b, p0, w, last, s); break;
-  }
+  if (rows < 1 || rows > 2048 || w < 1 || w > udt_panel_width(rows)) return hipErrorInvalidValue;
+  if (rows <= 64) launch_panel_t<1>(b, p0, w, last, s);
+  else if (rows <= 128) launch_panel_t<2>(b, p0, w, last, s);
+  else if (rows <= 256) launch_panel_t<4>(b, p0, w, last, s);
+  else if (rows <= 512) launch_panel_t<8>(b, p0, w, last, s);
+  else if (rows <= kPanelWideRows) launch_panel_t<16>(b, p0, w, last, s);
+  else
+    hipLaunchKernelGGL(udt_panel_tall_kernel<false>, dim3(b.count), dim3(512), (panel_lds<32, 8>()), s, b, p0, w,
+                       last);
   return hipGetLastError();
 }
 
@@ -919,19 +791,24 @@ hipError_t launch_udt_finish(const UdtBatch& b, hipStream_t s) {
   return hipGetLastError();
 }
 
-int udt_rows_class(int rows) { return udt_rows_per_thread(rows); }
+// Panels of one launch share the kernel: 16 waves and columns, or the tall form.
+int udt_rows_class(int rows) { return rows <= kPanelWideRows ? 1 : 8; }
 int udt_width_for(int rows) { return udt_panel_width(rows); }
 
 hipError_t launch_udt_panel_tab(const UdtBatch& b, int R, hipStream_t s) {
   if (!b.items || b.count < 1 || b.max_n < 1 || b.max_n > 2048) return hipErrorInvalidValue;
-  UdtBatch c = b;
-  c.n = b.max_n;          // sizes the dynamic LDS (per-item arrays of n entries)
-  switch (R) {
-    case 1: launch_panel_t<1, 16>(c, 0, 0, 0, s); break;
-    case 2: launch_panel_t<2, 16>(c, 0, 0, 0, s); break;
-    case 4: launch_panel_t<4, 16>(c, 0, 0, 0, s); break;
-    case 8: launch_panel_t<8, 8>(c, 0, 0, 0, s); break;
-    default: return hipErrorInvalidValue;
+  if (R == 1) {
+    // LDS for the tallest panel of the launch (an item of n sites in this class has at most
+    // min(n, 1024) rows)
+    const size_t lds = b.max_n <= 64 ? panel_lds<1, 16>()
+                     : b.max_n <= 128 ? panel_lds<2, 16>()
+                     : b.max_n <= 256 ? panel_lds<4, 16>()
+                     : b.max_n <= 512 ? panel_lds<8, 16>() : panel_lds<16, 16>();
+    hipLaunchKernelGGL(udt_panel_tab_kernel, dim3(b.count), dim3(1024), lds, s, b);
+  } else if (R == 8) {
+    hipLaunchKernelGGL(udt_panel_tall_kernel<true>, dim3(b.count), dim3(512), (panel_lds<32, 8>()), s, b, 0, 0, 0);
+  } else {
+    return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
@@ -1351,14 +1228,14 @@ hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s) {
 }
 
 hipError_t qr_kernels_init() {
-  const void* fns[] = {reinterpret_cast<const void*>(udt_panel_kernel<1, 16, false>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<2, 16, false>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<4, 16, false>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<8, 8, false>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<1, 16, true>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<2, 16, true>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<4, 16, true>),
-                       reinterpret_cast<const void*>(udt_panel_kernel<8, 8, true>),
+  const void* fns[] = {reinterpret_cast<const void*>(udt_panel_kernel<1>),
+                       reinterpret_cast<const void*>(udt_panel_kernel<2>),
+                       reinterpret_cast<const void*>(udt_panel_kernel<4>),
+                       reinterpret_cast<const void*>(udt_panel_kernel<8>),
+                       reinterpret_cast<const void*>(udt_panel_kernel<16>),
+                       reinterpret_cast<const void*>(udt_panel_tall_kernel<false>),
+                       reinterpret_cast<const void*>(udt_panel_tall_kernel<true>),
+                       reinterpret_cast<const void*>(udt_panel_tab_kernel),
                        reinterpret_cast<const void*>(rdivp_strip_kernel<false>),
                        reinterpret_cast<const void*>(rdivp_strip_kernel<true>),
                        reinterpret_cast<const void*>(rdivp_block_kernel<false, 16>),
