@@ -964,121 +964,122 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
   }
 }
 
-// Gd_b = Gs_b - C_b (Y_b R_b) on one 64 x 64 tile, for the previous window's flips with
-// its dense factor Y over positions wp .. wp + W - 1: C = (I - Gs)[:, wp:wp+W] and
-// R = Gs[wp:wp+W, :] are contiguous strips of the source copy (the update writes the other
-// copy, so no tile changes what another still reads).  The tile's slice of Z = Y R
-// (W x 64) is formed in LDS on the matrix cores; the rank-W product is computed
-// transposed, tile^T -= Z^T C^T, so accumulator element r of lane l is
-// G[r0 + l%16][c0 + row(l, r)]: quarter-waves touch 16 consecutive rows of a column.
+// Gd_b = Gs_b - C_b (Y_b R_b) on 64 x 64 tiles t0 .. t1 - 1 (down a column of tiles, then the
+// next column), for the previous window's flips with its dense factor Y over positions
+// wp .. wp + W - 1: C = (I - Gs)[:, wp:wp+W] and R = Gs[wp:wp+W, :] are contiguous strips of
+// the source copy (the update writes the other copy, so no tile changes what another still
+// reads).  The rank-W product is computed transposed, tile^T -= Z^T C^T, so accumulator element
+// r of lane l is G[r0 + l%16][c0 + row(l, r)]: quarter-waves touch 16 consecutive rows of a
+// column.
+//
+// What bounds a tile is memory latency (the strips were just written by other workgroups), so
+// every operand is loaded straight into the matrix-core registers, all in flight at once: wave w
+// owns rows 16 w .. (C's operand) and columns 16 w .. of Z = Y R (R's).  Only Z goes through
+// LDS, formed once per column of tiles, and the next tile's loads are issued before this tile's
+// products.  Against operands staged through LDS in turn, one tile after the other: 4.0 -> 3.6 us
+// for the one tile per workgroup of n = 256, 23 -> 18.5 us for the four of n = 1024 with two
+// flavours (a sweep of 32x32 sites 230 -> 216 ms).
 template <typename GT, int W>
-__device__ __forceinline__ void apply_tile(GT* __restrict__ Gd, const GT* __restrict__ Gs,
-                                          const int* __restrict__ Sp, const GT* __restrict__ Y, int n,
-                                          int wp, int tile, unsigned char* smem) {
-  typedef typename V4<GT>::type acc_t;
-  const int nt = (n + 63) >> 6;
-  const int b = tile / (nt * nt);
-  const int rem = tile - b * nt * nt;
-  const int r0 = (rem % nt) * 64, c0 = (rem / nt) * 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+struct ApplyTile {
+  typename V4<GT>::type acc[4];   // the tile of Gs: rows 16 wave + li, columns 16 j + row(lane, r)
+  GT cg[W / 4];                   // Gs[row][wp + 4 s + lk]
+};
+
+template <typename GT, int W>
+__device__ __forceinline__ void apply_load(ApplyTile<GT, W>& x, const GT* Gb, int n, int wp, int r0, int c0,
+                                           int lane, int wave) {
   const int li = lane & 15, lk = lane >> 4;
-  const size_t off = (size_t)b * n * n;
-  const GT* Gb = Gs + off;
-  GT* Gw = Gd + off;
-  const int rr0 = wave * 16;
-  const int grow = r0 + rr0 + li;
-  const int growc = grow < n ? grow : n - 1;
-  acc_t acc[4];
+  const int row = r0 + 16 * wave + li;
+  const size_t rowc = (size_t)(row < n ? row : n - 1);
 #pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int gcol = c0 + 16 * j + mfma_row<GT>(lane, r);
-      acc[j][r] = Gb[(size_t)growc + (size_t)(gcol < n ? gcol : n - 1) * n];
-    }
-  const int m = Sp[0];
-  if (m > 0) {
-    GT* Ys = reinterpret_cast<GT*>(smem);   // W x W column-major: Ys[l * W + k] = Y[k][l]
-    GT* Rs = Ys + W * W;                     // W x 64  [k][col]
-    GT* Zs = Rs + W * 64;                    // W x 65  [k][col]
-    GT* Cs = Zs + W * 65;                    // 64 x W+1 [row][k]
-    {
-      // R[k][c0 + cc] = Gs[wp + k][c0 + cc]: lane = k, cc = wave + 4 q
-      const int k = wp + (lane < W ? lane : W - 1);
-      const size_t ko = (size_t)(k < n ? k : n - 1);
-      GT v[16];
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int gc = c0 + wave + 4 * q;
-        v[q] = Gb[ko + (size_t)(gc < n ? gc : n - 1) * n];
-      }
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int gc = c0 + wave + 4 * q;
-        if (lane < W) Rs[lane * 64 + wave + 4 * q] = gc < n ? v[q] : GT(0);
-      }
-    }
-    {
-      // C[r0 + rr][k] = delta - Gs[r0 + rr][wp + k]: lane = rr, k = wave + 4 q
-      constexpr int QC = W / 4;
-      const int gr = r0 + lane;
-      const int grc = gr < n ? gr : n - 1;
-      GT v[QC];
-#pragma unroll
-      for (int q = 0; q < QC; q++) {
-        const int k = wp + wave + 4 * q;
-        v[q] = Gb[(size_t)grc + (size_t)(k < n ? k : n - 1) * n];
-      }
-#pragma unroll
-      for (int q = 0; q < QC; q++) {
-        const int k = wave + 4 * q;
-        Cs[lane * (W + 1) + k] = gr < n ? (gr == wp + k ? GT(1) : GT(0)) - v[q] : GT(0);
-      }
-    }
-    {
-      // Y (row-major W x W in global): Ys[l * W + k] = Y[k][l]; lane = l, k = wave + 4 q
-      constexpr int QY = W / 4;
-      const int lc = lane < W ? lane : W - 1;
-      GT v[QY];
-#pragma unroll
-      for (int q = 0; q < QY; q++) v[q] = Y[(size_t)b * W * W + (size_t)(wave + 4 * q) * W + lc];
-#pragma unroll
-      for (int q = 0; q < QY; q++)
-        if (lane < W) Ys[lane * W + wave + 4 * q] = v[q];
-    }
-    __syncthreads();
-    // Z[:, 16 wave : 16 wave + 16] = Y R[:, same columns]
-#pragma unroll
-    for (int i0 = 0; i0 < W; i0 += 16) {
-      acc_t z = {0, 0, 0, 0};
-#pragma unroll
-      for (int k0 = 0; k0 < W; k0 += 4) {
-        const GT av = Ys[(k0 + lk) * W + i0 + li];        // Y[i0 + li][k0 + lk]
-        const GT bv = Rs[(k0 + lk) * 64 + 16 * wave + li];  // R[k0 + lk][16 wave + li]
-        z = mfma16(av, bv, z);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) Zs[(i0 + mfma_row<GT>(lane, r)) * 65 + 16 * wave + li] = z[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k0 = 0; k0 < W; k0 += 4) {
-      const int k = k0 + lk;
-      const GT bv = Cs[(rr0 + li) * (W + 1) + k];          // C^T[k][row]
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const GT av = -Zs[k * 65 + 16 * j + li];           // Z^T[col][k]
-        acc[j] = mfma16(av, bv, acc[j]);
-      }
-    }
+  for (int s = 0; s < W / 4; s++) {
+    const int k = wp + 4 * s + lk;
+    x.cg[s] = Gb[rowc + (size_t)(k < n ? k : n - 1) * n];
   }
 #pragma unroll
   for (int j = 0; j < 4; j++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int gcol = c0 + 16 * j + mfma_row<GT>(lane, r);
-      if (grow < n && gcol < n) Gw[(size_t)grow + (size_t)gcol * n] = acc[j][r];
+      x.acc[j][r] = Gb[rowc + (size_t)(gcol < n ? gcol : n - 1) * n];
     }
+}
+
+template <typename GT, int W>
+__device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __restrict__ Gs,
+                                           const int* __restrict__ Sp, const GT* __restrict__ Y, int n,
+                                           int wp, int t0, int t1, unsigned char* smem) {
+  typedef typename V4<GT>::type acc_t;
+  constexpr int KS = W / 4, CT = W / 16;
+  const int nt = (n + 63) >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  GT* Zs = reinterpret_cast<GT*>(smem);     // W x 65  [k][col]
+  const int m = Sp[0];
+  ApplyTile<GT, W> cur, nxt;
+  {
+    const int b = t0 / (nt * nt), rem = t0 - b * nt * nt;
+    apply_load<GT, W>(cur, Gs + (size_t)b * n * n, n, wp, (rem % nt) * 64, (rem / nt) * 64, lane, wave);
+  }
+  int zcol = -1;                            // the column of tiles Zs holds (counted over the blocks)
+  for (int t = t0; t < t1; t++) {
+    const int b = t / (nt * nt), rem = t - b * nt * nt;
+    const int r0 = (rem % nt) * 64, c0 = (rem / nt) * 64;
+    const size_t off = (size_t)b * n * n;
+    const GT* Gb = Gs + off;
+    GT* Gw = Gd + off;
+    const bool newz = t / nt != zcol;
+    GT rv[KS], yv[CT][KS];
+    const int zc = c0 + 16 * wave + li;
+    if (newz) {
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const int k = wp + 4 * s + lk;
+        rv[s] = Gb[(size_t)(k < n ? k : n - 1) + (size_t)(zc < n ? zc : n - 1) * n];
+      }
+#pragma unroll
+      for (int i = 0; i < CT; i++)
+#pragma unroll
+        for (int s = 0; s < KS; s++) yv[i][s] = Y[(size_t)b * W * W + (size_t)(16 * i + li) * W + 4 * s + lk];
+    }
+    if (t + 1 < t1) {
+      const int b1 = (t + 1) / (nt * nt), rem1 = t + 1 - b1 * nt * nt;
+      apply_load<GT, W>(nxt, Gs + (size_t)b1 * n * n, n, wp, (rem1 % nt) * 64, (rem1 / nt) * 64, lane, wave);
+    }
+    if (m > 0) {
+      if (newz) {
+        if (zcol >= 0) __syncthreads();     // the waves have read the previous column's Z
+        // Z[:, 16 wave : 16 wave + 16] = Y R[:, same columns]
+#pragma unroll
+        for (int i = 0; i < CT; i++) {
+          acc_t z = {0, 0, 0, 0};
+#pragma unroll
+          for (int s = 0; s < KS; s++) z = mfma16(yv[i][s], zc < n ? rv[s] : GT(0), z);
+#pragma unroll
+          for (int r = 0; r < 4; r++) Zs[(16 * i + mfma_row<GT>(lane, r)) * 65 + 16 * wave + li] = z[r];
+        }
+        __syncthreads();
+        zcol = t / nt;
+      }
+      const int row = r0 + 16 * wave + li;
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const int k = 4 * s + lk;
+        const GT bv = row < n ? (row == wp + k ? GT(1) : GT(0)) - cur.cg[s] : GT(0);   // C^T[k][row]
+#pragma unroll
+        for (int j = 0; j < 4; j++) cur.acc[j] = mfma16(-Zs[k * 65 + 16 * j + li], bv, cur.acc[j]);
+      }
+    }
+    const int grow = r0 + 16 * wave + li;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int gcol = c0 + 16 * j + mfma_row<GT>(lane, r);
+        if (grow < n && gcol < n) Gw[(size_t)grow + (size_t)gcol * n] = cur.acc[j][r];
+      }
+    cur = nxt;
+  }
 }
 
 // One launch per window: workgroup 0 runs the window (decisions on the block formed from
@@ -1091,14 +1092,16 @@ __global__ __launch_bounds__(256) void window_kernel(WindowArgs<GT> a) {
     window_role<GT, FLV, W>(a, smem);
     return;
   }
-  apply_tile<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, (int)blockIdx.x - 1, smem);
+  const int t = (int)blockIdx.x - 1;
+  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, t, t + 1, smem);
 }
 
 // The last window's application alone.
 template <typename GT, int W>
 __global__ __launch_bounds__(256) void window_apply_kernel(WindowArgs<GT> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  apply_tile<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, (int)blockIdx.x, smem);
+  const int t = (int)blockIdx.x;
+  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, t, t + 1, smem);
 }
 
 // Bounded wait until *p >= v (device scope); false when the bound is reached.
@@ -1114,8 +1117,8 @@ __device__ __forceinline__ bool wait_at_least(const unsigned long long* p, unsig
 // One launch per slice.  Workgroup 0 runs windows 0 .. nw - 1 back to back, as in
 // window_kernel, pipelined (SliceCtl): window k's block operands were prefetched during window
 // k - 1 once every application of window k - 2 was done (window k reads their output copy),
-// and window k - 1's factor is published once window k's block is formed.  Workgroup 1 + i applies window j to tiles
-// i, i + napply, ... once window j is published and every application of window j - 1 is
+// and window k - 1's factor is published once window k's block is formed.  Workgroup 1 + i applies window j to its
+// own run of tiles once window j is published and every application of window j - 1 is
 // done (whose source copy window j's application overwrites).  Every wait is bounded; a wait
 // that gives up counts a device error and the launch still ends.  All workgroups are resident
 // at once (one per CU, 1 + napply <= 129), and a workgroup waits only for work that needs no
@@ -1185,7 +1188,8 @@ __global__ __launch_bounds__(256) void window_slice_kernel(WindowSlice<GT> s) {
     return;
   }
   const int nt = (s.a.n + 63) >> 6;
-  const int tiles = FLV * nt * nt;
+  const int tiles = FLV * nt * nt, per = (tiles + s.napply - 1) / s.napply;
+  const int t0 = ((int)blockIdx.x - 1) * per, t1 = t0 + per < tiles ? t0 + per : tiles;
   for (int j = 0; j < s.nw; j++) {
     if (tid == 0) {
       bool ok = wait_at_least(ready + j, e + 1, limit);
@@ -1194,11 +1198,9 @@ __global__ __launch_bounds__(256) void window_slice_kernel(WindowSlice<GT> s) {
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
-    for (int t = (int)blockIdx.x - 1; t < tiles; t += s.napply) {
-      apply_tile<GT, W>(s.B[(j + 1) & 1], s.B[j & 1], s.S + (j & 1) * (W + 1), s.Y + (j & 1) * ysz, s.a.n,
-                        j * W, t, smem);
-      __syncthreads();
-    }
+    if (t0 < t1)
+      apply_tiles<GT, W>(s.B[(j + 1) & 1], s.B[j & 1], s.S + (j & 1) * (W + 1), s.Y + (j & 1) * ysz, s.a.n,
+                         j * W, t0, t1, smem);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
     if (tid == 0) {
@@ -1210,7 +1212,7 @@ __global__ __launch_bounds__(256) void window_slice_kernel(WindowSlice<GT> s) {
 
 template <typename GT, int W>
 constexpr size_t apply_lds() {
-  return sizeof(GT) * ((size_t)W * W + W * 64 + W * 65 + 64 * (W + 1));
+  return sizeof(GT) * (size_t)W * 65;
 }
 
 // Sites per window (delay_depth selects 16, 32 or 64 explicitly).  Per-flip work and the
@@ -1255,7 +1257,7 @@ __global__ __launch_bounds__(256) void window_multi_kernel(const WindowArgs<GT>*
   const int nt = (a.n + 63) / 64;
   const int tile = (int)blockIdx.x - 1;
   if (tile >= a.flv * nt * nt) return;
-  apply_tile<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile, smem);
+  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile, tile + 1, smem);
 }
 
 template <int W>
