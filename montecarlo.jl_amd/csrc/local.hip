@@ -232,69 +232,27 @@ __device__ __forceinline__ void window_block_direct(const WindowArgs<GT>& a, dou
   }
 }
 
+// The products of the block from its operands in LDS: block b's G[w, w], G[w, wp], G[wp, w] at M0 +
+// mats b W LD (one after the other), its previous factor at Y0 + ymats b W LD; corr: there were flips.
 template <typename GT, int FLV, int W>
-__device__ __forceinline__ void window_block_staged(const WindowArgs<GT>& a, double* Bn, GT* St, GT* Zw, int Wn,
-                                                    int tid, int lane, int wave,
-                                                    const SliceCtl<GT>* sc = nullptr) {
+__device__ __forceinline__ void window_block_form(double* Bn, const GT* M0, int mats, const GT* Y0, int ymats,
+                                                  bool corr, GT* Zw, int lane, int wave) {
   typedef typename V4<GT>::type acc_t;
-  constexpr int CT = W / 16, KS = W / 4, LD = W + 1, WW = W * W, QM = WW / 256;
-  static_assert(WW % 256 == 0, "staging assumes whole passes of 256 threads per matrix");
-  const int n = a.n, w0 = a.w0, wp = a.wp;
-  const size_t nn = (size_t)n * n;
+  constexpr int CT = W / 16, KS = W / 4, LD = W + 1;
   const int li = lane & 15, lk = lane >> 4;
-  const bool corr = a.Yp != nullptr;
-  const int mp = corr ? a.Sp[0] : 0;
-  // St[(4 b + mat) W LD + c LD + r]: mat 0 = G[w, w], 1 = G[w, wp], 2 = G[wp, w]
-  // (column-major, [c][r]); mat 3 = previous factor (row-major, [p][q])
-  const bool lds_in = sc != nullptr && sc->pf_in;
-  if (!lds_in) {
-  GT v[FLV][4][QM];
-#pragma unroll
-  for (int b = 0; b < FLV; b++) {
-    const GT* Gb = a.G + (size_t)b * nn;
-#pragma unroll
-    for (int q = 0; q < QM; q++) {
-      const int idx = tid + 256 * q;
-      const int r = idx % W, c = idx / W;
-      const int rw = w0 + (r < Wn ? r : Wn - 1), cw = w0 + (c < Wn ? c : Wn - 1);
-      const int rp = wp + r < n ? wp + r : n - 1, cp = wp + c < n ? wp + c : n - 1;
-      v[b][0][q] = Gb[(size_t)rw + (size_t)cw * n];
-      if (corr) {
-        v[b][1][q] = Gb[(size_t)rw + (size_t)cp * n];
-        v[b][2][q] = Gb[(size_t)rp + (size_t)cw * n];
-        v[b][3][q] = a.Yp[(size_t)b * WW + idx];
-      }
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < FLV; b++)
-#pragma unroll
-    for (int q = 0; q < QM; q++) {
-      const int idx = tid + 256 * q;
-      const int r = idx % W, c = idx / W;
-      GT* Sb = St + (size_t)(4 * b) * W * LD + c * LD + r;
-      Sb[0] = v[b][0][q];
-      if (corr) {
-        Sb[W * LD] = v[b][1][q];
-        Sb[2 * W * LD] = v[b][2][q];
-        Sb[3 * W * LD] = v[b][3][q];
-      }
-    }
-  __syncthreads();
-  }
   for (int unit = wave; unit < FLV * CT; unit += 4) {
     const int b = unit / CT, ci = unit - b * CT;
-    const GT* Bs = lds_in ? sc->pf + (size_t)(3 * b) * W * LD : St + (size_t)(4 * b) * W * LD;
+    const GT* Bs = M0 + (size_t)(mats * b) * W * LD;
     const GT* Ps = Bs + W * LD;
     const GT* Qs = Bs + 2 * W * LD;
-    const GT* Ys = lds_in ? sc->yl + (size_t)b * W * LD : Bs + 3 * W * LD;
+    const GT* Ys = Y0 + (size_t)(ymats * b) * W * LD;
     const int cc = ci * 16 + li;
     acc_t o[CT];
 #pragma unroll
     for (int t = 0; t < CT; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) o[t][r] = Bs[cc * LD + t * 16 + mfma_row<GT>(lane, r)];
-    if (corr && mp > 0) {
+    if (corr) {
       acc_t z[CT];
 #pragma unroll
       for (int t = 0; t < CT; t++) {
@@ -337,6 +295,58 @@ __device__ __forceinline__ void window_block_staged(const WindowArgs<GT>& a, dou
 #pragma unroll
       for (int r = 0; r < 4; r++) Bb[cc * LD + t * 16 + mfma_row<GT>(lane, r)] = (double)o[t][r];
   }
+}
+
+template <typename GT, int FLV, int W>
+__device__ __forceinline__ void window_block_staged(const WindowArgs<GT>& a, double* Bn, GT* St, GT* Zw, int Wn,
+                                                    int tid, int lane, int wave,
+                                                    const SliceCtl<GT>* sc = nullptr) {
+  constexpr int LD = W + 1, WW = W * W, QM = WW / 256;
+  static_assert(WW % 256 == 0, "staging assumes whole passes of 256 threads per matrix");
+  const int n = a.n, w0 = a.w0, wp = a.wp;
+  const size_t nn = (size_t)n * n;
+  const bool corr = a.Yp != nullptr;
+  const int mp = corr ? a.Sp[0] : 0;
+  // St[(4 b + mat) W LD + c LD + r]: mat 0 = G[w, w], 1 = G[w, wp], 2 = G[wp, w]
+  // (column-major, [c][r]); mat 3 = previous factor (row-major, [p][q])
+  const bool lds_in = sc != nullptr && sc->pf_in;
+  if (!lds_in) {
+  GT v[FLV][4][QM];
+#pragma unroll
+  for (int b = 0; b < FLV; b++) {
+    const GT* Gb = a.G + (size_t)b * nn;
+#pragma unroll
+    for (int q = 0; q < QM; q++) {
+      const int idx = tid + 256 * q;
+      const int r = idx % W, c = idx / W;
+      const int rw = w0 + (r < Wn ? r : Wn - 1), cw = w0 + (c < Wn ? c : Wn - 1);
+      const int rp = wp + r < n ? wp + r : n - 1, cp = wp + c < n ? wp + c : n - 1;
+      v[b][0][q] = Gb[(size_t)rw + (size_t)cw * n];
+      if (corr) {
+        v[b][1][q] = Gb[(size_t)rw + (size_t)cp * n];
+        v[b][2][q] = Gb[(size_t)rp + (size_t)cw * n];
+        v[b][3][q] = a.Yp[(size_t)b * WW + idx];
+      }
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < FLV; b++)
+#pragma unroll
+    for (int q = 0; q < QM; q++) {
+      const int idx = tid + 256 * q;
+      const int r = idx % W, c = idx / W;
+      GT* Sb = St + (size_t)(4 * b) * W * LD + c * LD + r;
+      Sb[0] = v[b][0][q];
+      if (corr) {
+        Sb[W * LD] = v[b][1][q];
+        Sb[2 * W * LD] = v[b][2][q];
+        Sb[3 * W * LD] = v[b][3][q];
+      }
+    }
+  __syncthreads();
+  }
+  if (lds_in) window_block_form<GT, FLV, W>(Bn, sc->pf, 3, sc->yl, 1, mp > 0, Zw, lane, wave);
+  else window_block_form<GT, FLV, W>(Bn, St, 4, St + 3 * W * LD, 4, mp > 0, Zw, lane, wave);
 }
 
 template <typename GT, int FLV, int W>
@@ -964,31 +974,506 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
   }
 }
 
-// Gd_b = Gs_b - C_b (Y_b R_b) on 64 x 64 tiles t0 .. t1 - 1 (down a column of tiles, then the
-// next column), for the previous window's flips with its dense factor Y over positions
-// wp .. wp + W - 1: C = (I - Gs)[:, wp:wp+W] and R = Gs[wp:wp+W, :] are contiguous strips of
-// the source copy (the update writes the other copy, so no tile changes what another still
-// reads).  The rank-W product is computed transposed, tile^T -= Z^T C^T, so accumulator element
-// r of lane l is G[r0 + l%16][c0 + row(l, r)]: quarter-waves touch 16 consecutive rows of a
-// column.
+// ---------------------------------------------------------------------------------------
+// Windows of 16 sites.  One wave runs the decisions, a second builds the factor beside it, and
+// neither moves a row or a column of the block through LDS:
+//  * Every 16-lane row of a wave holds one 16 x 16 matrix of one flavour block, a matrix row
+//    (or column) per lane, all 16 entries in registers.  A rank-1 update adds a multiple of
+//    row t of the matrix, and row t is lane t's registers: v_fmac_f64 takes it through
+//    row_newbcast, one instruction per column (row_flip, row_add, row_update).
+//  * The decision wave keeps each flavour's block twice, by rows in the even and by columns in
+//    the odd 16-lane row, so that an exchange of two rows of lanes (swap16) gives every lane
+//    both G[r][t] and G[t][r] for its diagonal entry.
+//  * The factor wave keeps, per flavour, the block B and P = I + Y B0 by rows in the even and
+//    Q = I - (I - B0) Y and Y in the odd 16-lane row (B0: the window's block before its flips).
+//    Then C = C0 P and R = Q R0, so a flip at t with gamma is
+//      Y += gamma P[:,t] Q[t,:],  P += gamma P[:,t] B[t,:],
+//      Q -= gamma u Q[t,:],       B -= gamma u B[t,:],      u = e_t - B[:,t]:
+//    multiples of the same two broadcast rows.  It needs only t and gamma of a flip, and Y comes
+//    out over window positions, with exact zeros in the rows and columns of rejected sites.
+// What bounds a window is the instruction stream of these two lone waves.
+// ---------------------------------------------------------------------------------------
+
+typedef double d16 __attribute__((ext_vector_type(16)));
+
+// Updates by row t of the matrix in x (lane t's registers, in every 16-lane row of the wave).  A
+// broadcast lane is part of the instruction and t, though uniform, is known only at run time: the
+// block jumps to case t of a table of straight-line cases.  The matrices sit in fixed registers,
+// x in v[96:127] and y in v[64:95], so that the block names their parts and updates them in place
+// (a switch around single updates made the compiler copy all 16 entries twice per flip).  The
+// wait states before the jump cover a register written just before the block.
+#define DQMC_ROW1(a, b, c, d, t) "v_fmac_f64_dpp v[" #a ":" #b "], v[" #c ":" #d "], %[l] row_newbcast:" #t \
+                                 " row_mask:0xf bank_mask:0xf\n\t"
+#define DQMC_ROW_X(t) \
+  DQMC_ROW1(96, 97, 96, 97, t) DQMC_ROW1(98, 99, 98, 99, t) DQMC_ROW1(100, 101, 100, 101, t) \
+  DQMC_ROW1(102, 103, 102, 103, t) DQMC_ROW1(104, 105, 104, 105, t) DQMC_ROW1(106, 107, 106, 107, t) \
+  DQMC_ROW1(108, 109, 108, 109, t) DQMC_ROW1(110, 111, 110, 111, t) DQMC_ROW1(112, 113, 112, 113, t) \
+  DQMC_ROW1(114, 115, 114, 115, t) DQMC_ROW1(116, 117, 116, 117, t) DQMC_ROW1(118, 119, 118, 119, t) \
+  DQMC_ROW1(120, 121, 120, 121, t) DQMC_ROW1(122, 123, 122, 123, t) DQMC_ROW1(124, 125, 124, 125, t) \
+  DQMC_ROW1(126, 127, 126, 127, t)
+#define DQMC_ROW_Y(t) \
+  DQMC_ROW1(64, 65, 96, 97, t) DQMC_ROW1(66, 67, 98, 99, t) DQMC_ROW1(68, 69, 100, 101, t) \
+  DQMC_ROW1(70, 71, 102, 103, t) DQMC_ROW1(72, 73, 104, 105, t) DQMC_ROW1(74, 75, 106, 107, t) \
+  DQMC_ROW1(76, 77, 108, 109, t) DQMC_ROW1(78, 79, 110, 111, t) DQMC_ROW1(80, 81, 112, 113, t) \
+  DQMC_ROW1(82, 83, 114, 115, t) DQMC_ROW1(84, 85, 116, 117, t) DQMC_ROW1(86, 87, 118, 119, t) \
+  DQMC_ROW1(88, 89, 120, 121, t) DQMC_ROW1(90, 91, 122, 123, t) DQMC_ROW1(92, 93, 124, 125, t) \
+  DQMC_ROW1(94, 95, 126, 127, t)
+// jump to case t of the table that follows, `size` bytes per case
+#define DQMC_ROW_JUMP(size) \
+  "s_nop 1\n\ts_mul_i32 s42, %[t], " #size "\n\ts_getpc_b64 s[40:41]\n.Lrow_pc%=:\n\t" \
+  "s_add_u32 s40, s40, s42\n\ts_addc_u32 s41, s41, 0\n\ts_add_u32 s40, s40, .Lrow_tab%=-.Lrow_pc%=\n\t" \
+  "s_addc_u32 s41, s41, 0\n\ts_setpc_b64 s[40:41]\n.Lrow_tab%=:\n\t"
+#define DQMC_CASES16(M) \
+  M(0, 96, 97) M(1, 98, 99) M(2, 100, 101) M(3, 102, 103) M(4, 104, 105) M(5, 106, 107) M(6, 108, 109) M(7, 110, 111) \
+  M(8, 112, 113) M(9, 114, 115) M(10, 116, 117) M(11, 118, 119) M(12, 120, 121) M(13, 122, 123) M(14, 124, 125) \
+  M(15, 126, 127)
+
+// gam = gq of lane t of this 16-lane row; x[c] += gam v x[c][lane t], c = 0 .. 15; x[t] += gam w.
+__device__ __forceinline__ void row_flip(d16& x, double gq, double v, double w, int t, double& gam) {
+  double l;
+#define DQMC_FLIP(t, a, b)                                                                                  \
+  "v_mov_b64_dpp %[g], %[gq] row_newbcast:" #t " row_mask:0xf bank_mask:0xf\n\tv_mul_f64 %[l], %[g], %[v]\n\t" \
+  DQMC_ROW_X(t) "v_fma_f64 v[" #a ":" #b "], %[g], %[w], v[" #a ":" #b "]\n\ts_branch .Lrow_end%=\n\t"
+  asm volatile(DQMC_ROW_JUMP(156) DQMC_CASES16(DQMC_FLIP) ".Lrow_end%=:"
+               : "+{v[96:127]}"(x), [g] "=&v"(gam), [l] "=&v"(l)
+               : [gq] "v"(gq), [v] "v"(v), [w] "v"(w), [t] "s"(t)
+               : "s40", "s41", "s42", "scc");
+#undef DQMC_FLIP
+}
+// y[c] += l x[c][lane t], c = 0 .. 15.
+__device__ __forceinline__ void row_add(d16& y, d16& x, double l, int t) {
+#define DQMC_ADD(t, a, b) DQMC_ROW_Y(t) "s_branch .Lrow_end%=\n\t"
+  asm volatile(DQMC_ROW_JUMP(132) DQMC_CASES16(DQMC_ADD) ".Lrow_end%=:"
+               : "+{v[64:95]}"(y), "+{v[96:127]}"(x)
+               : [l] "v"(l), [t] "s"(t)
+               : "s40", "s41", "s42", "scc");
+#undef DQMC_ADD
+}
+// x[c] += l x[c][lane t], c = 0 .. 15.
+__device__ __forceinline__ void row_update(d16& x, double l, int t) {
+#define DQMC_UPD(t, a, b) DQMC_ROW_X(t) "s_branch .Lrow_end%=\n\t"
+  asm volatile(DQMC_ROW_JUMP(132) DQMC_CASES16(DQMC_UPD) ".Lrow_end%=:"
+               : "+{v[96:127]}"(x)
+               : [l] "v"(l), [t] "s"(t)
+               : "s40", "s41", "s42", "scc");
+#undef DQMC_UPD
+}
+#undef DQMC_ROW1
+#undef DQMC_ROW_X
+#undef DQMC_ROW_Y
+#undef DQMC_ROW_JUMP
+#undef DQMC_CASES16
+
+// Both 16-lane rows of a pair get x of the even one (ev) and of the odd one (od), lane by lane.
+__device__ __forceinline__ void swap16(double x, double& ev, double& od) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(x), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(x), false, false);
+  ev = __hiloint2double((int)hi[0], (int)lo[0]);
+  od = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// The same for the two halves of the wave.
+__device__ __forceinline__ void swap32(double x, double& first, double& second) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(x), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(x), false, false);
+  first = __hiloint2double((int)hi[0], (int)lo[0]);
+  second = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// LDS of a 16-site window: the block; the staged operands (slices: the prefetched operands and the
+// factor); the flips published to the factor wave; results; the uniforms and field of `nu` sites.
+struct Win16Pub {
+  double gam[16][2];     // per flip and flavour block
+  int site[16];
+  int flips, fin;        // flips published; final count (-1 while deciding)
+  int m, pad;            // the last finished window's flips
+};
+template <typename GT, int FLV>
+constexpr size_t win16_lds(int nu) {
+  return (size_t)FLV * 16 * 17 * 8 + (size_t)4 * FLV * 16 * 17 * sizeof(GT) +
+         (sizeof(GT) == 4 ? (size_t)4 * 16 * 17 * 4 : 0) + sizeof(Win16Pub) + (size_t)nu * 9 + 16;
+}
+
+struct Win16Tally {
+  int used, flips, neg, ties;
+};
+
+// The decisions of one window (one wave).  Bn: the block, [f][column][row] with leading dimension
+// 17; U: the window's uniforms, U[k] for the k-th one used (k <= kmax); cf: site r's field.
+// Rounds: every undecided site's proposal is formed at once from the current diagonals; the sites
+// before the first accepted one are rejected with exactly the values a site-by-site loop would
+// form, that one is flipped, and the next round starts after it.  Uniforms go to the proposals
+// with p <= 1 in site order; a site's uniform stays the same one while that set of undecided
+// sites does, so it is gathered again only when the set changed.
+template <typename GT, int FLV>
+__device__ __forceinline__ void decide16(const WindowArgs<GT>& a, const double* Bn, Win16Pub* pub, const double* U,
+                                         int kmax, int cf, int w0, int Wn, long long log0, int lane,
+                                         Win16Tally& tl) {
+  const int f = lane >> 5, fb = FLV > 1 ? f : 0, r = lane & 15;
+  const bool bycol = (lane & 16) != 0;
+  const int rc = r < Wn ? r : Wn - 1;
+  const double* Bf = Bn + (size_t)fb * 16 * 17;
+  d16 g;
+  double dg = Bf[rc * 17 + rc];
+  {
+    const double* B0 = Bf + (bycol ? r * 17 : r);
+    const int step = bycol ? 1 : 17;
+#pragma unroll
+    for (int c = 0; c < 16; c++) g[c] = B0[c * step];
+  }
+  if (Wn < 16) {                                 // rows and columns beyond the lattice
+#pragma unroll
+    for (int c = 0; c < 16; c++) g[c] = r < Wn && c < Wn ? g[c] : 0.0;
+  }
+  const double df0 = a.d_first[0], df1 = a.d_first[1], ds0 = a.d_second[0], ds1 = a.d_second[1];
+  const double bw0 = a.bweight[0], bw1 = a.bweight[1];
+  const double d0 = FLV > 1 && f ? ds0 : df0, d1 = FLV > 1 && f ? ds1 : df1;
+  const double d = cf > 0 ? d1 : d0, bw = cf > 0 ? bw1 : bw0;
+  const unsigned int below = (1u << r) - 1u;
+  unsigned int und = (1u << Wn) - 1u, need_prev = 0, accepted = 0;
+  int m = 0, used = 0, shown = 0;
+  double p_r = 0.0, u_r = 0.0, u = 0.0;
+  while (und) {
+    double R, R0, R1, p;
+    {
+#pragma clang fp contract(off)
+      R = 1.0 + d * (1.0 - dg);
+      if constexpr (FLV > 1) {
+        swap32(R, R0, R1);
+        p = R0 * R1;
+      } else {
+        const double det = R * R;
+        p = bw * det;
+      }
+    }
+    const unsigned int big = (unsigned int)__ballot(p > 1.0);
+    const unsigned int need = ~big & und;
+    if (need != (need_prev & und)) {
+      const int k = used + __popc(need & below);
+      u = U[k < kmax ? k : kmax];
+    }
+    need_prev = need;
+    if (m != shown) {                            // the last flip's site and gammas are written by now
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      if (lane == 0) __hip_atomic_store(&pub->flips, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      shown = m;
+    }
+    const unsigned int accm = (big | (unsigned int)__ballot(u < p)) & und;
+    const unsigned int dec = accm ? (und & (((accm & (0u - accm)) << 1) - 1u)) : und;   // decided this round
+    const bool mine = ((dec >> r) & 1u) != 0;
+    p_r = mine ? p : p_r;
+    u_r = mine ? u : u_r;
+    used += __popc(need & dec);
+    und &= ~dec;
+    if (!accm) break;
+    const int t = __builtin_ctz(accm);
+    accepted |= accm & (0u - accm);
+    // the flip: by rows G[r][c] -= gam u_r G[t][c], by columns G[k][r] -= gam u_k G[t][r], with
+    // u = e_t - G[:,t] (by columns the 1 of u_t is entry t's own term)
+    const double gq = gamma_of(d, R);            // every site's gamma
+    double grt, gtr, gam;                        // G[r][t], G[t][r]
+    swap16(g[t], grt, gtr);
+    const double e = grt - (r == t ? 1.0 : 0.0);
+    row_flip(g, gq, bycol ? gtr : e, bycol ? -gtr : 0.0, t, gam);
+    dg = fma(gam * e, gtr, dg);
+    if ((lane & 31) == 0) pub->gam[m][f] = gam;
+    if (lane == 0) pub->site[m] = t;
+    m++;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (lane == 0) {
+    __hip_atomic_store(&pub->flips, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_store(&pub->fin, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  // negative probabilities and ties of the window's sites
+  const unsigned int win = (1u << Wn) - 1u;
+  const bool tie = p_r > 1.0 ? (p_r - 1.0 < 1e-12) : (fabs(u_r - p_r) < 1e-12);
+  tl.neg += __popc((unsigned int)__ballot(p_r < 0.0) & win);
+  tl.ties += __popc((unsigned int)__ballot(tie) & win);
+  tl.used += used;
+  tl.flips += m;
+  if (lane == 0) pub->m = m;
+  if (lane < Wn) {
+    const bool acc = ((accepted >> lane) & 1u) != 0;
+    if (a.dec_log && log0 + lane < a.log_cap) {
+      a.dec_log[log0 + lane] = (unsigned char)acc;
+      if (a.p_log) a.p_log[log0 + lane] = p_r;
+    }
+    if (acc) a.conf[w0 + lane] = (int8_t)(-cf);
+  }
+}
+
+// The factor of one window (one wave, beside decide16): Y to global memory and, for slices, to LDS
+// (yl, leading dimension 17), the flip count to S.  The wait for a flip is bounded; giving up
+// leaves Y wrong, so it is counted as a device error that the host reports.
+template <typename GT, int FLV>
+__device__ __forceinline__ void factor16(const WindowArgs<GT>& a, const double* Bn, Win16Pub* pub, int Wn, int lane,
+                                         GT* Y, int* S, GT* yl) {
+  const int f = lane >> 5, fb = FLV > 1 ? f : 0, r = lane & 15;
+  const bool odd = (lane & 16) != 0;
+  const double* Bf = Bn + (size_t)fb * 16 * 17;
+  d16 x, y;
+#pragma unroll
+  for (int c = 0; c < 16; c++) {
+    const double b = Bf[c * 17 + r], e = r == c ? 1.0 : 0.0;
+    x[c] = odd ? e : (r < Wn && c < Wn ? b : 0.0);
+    y[c] = odd ? 0.0 : e;
+  }
+  int k = 0;
+  long long polls = 0;
+  for (;;) {
+    int avail = __hip_atomic_load(&pub->flips, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (avail <= k) {
+      const int fin = __hip_atomic_load(&pub->fin, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (fin < 0) {
+        if (++polls > a.wait_limit) {
+          if (lane == 0) atomicAdd(reinterpret_cast<unsigned long long*>(&a.ctr->device_errors), 1ull);
+          break;
+        }
+        continue;
+      }
+      if (fin <= k) break;
+    }
+    const int t = __builtin_amdgcn_readfirstlane(pub->site[k]);
+    const double gam = pub->gam[k][fb];
+    double brt, prt, unused;                     // B[r][t], P[r][t]
+    swap16(x[t], brt, unused);
+    swap16(y[t], prt, unused);
+    row_add(y, x, gam * prt, t);
+    row_update(x, gam * (brt - (r == t ? 1.0 : 0.0)), t);
+    k++;
+  }
+  if (odd && f < FLV) {
+    GT* Yr = Y + (size_t)f * 256 + r * 16;
+#pragma unroll
+    for (int c = 0; c < 16; c++) Yr[c] = (GT)y[c];
+    if (yl) {
+      GT* yr = yl + (size_t)f * 16 * 17 + r * 17;
+#pragma unroll
+      for (int c = 0; c < 16; c++) yr[c] = (GT)y[c];
+    }
+  }
+  if (lane == 0) S[0] = k;
+}
+
+// One 16-site window of one launch (window_kernel, window_multi_kernel): the block from the source
+// copy and the previous window's factor, then decisions (wave 0) and factor (wave 2).
+template <typename GT, int FLV>
+__device__ __forceinline__ void window16_role(const WindowArgs<GT>& a, unsigned char* smem) {
+  double* Bn = reinterpret_cast<double*>(smem);
+  GT* St = reinterpret_cast<GT*>(Bn + FLV * 16 * 17);
+  GT* Zw = St + 4 * FLV * 16 * 17;
+  Win16Pub* pub = reinterpret_cast<Win16Pub*>(Zw + (sizeof(GT) == 4 ? 4 * 16 * 17 : 0));
+  double* U = reinterpret_cast<double*>(pub + 1);
+  const int n = a.n, w0 = a.w0, Wn = n - w0 < 16 ? n - w0 : 16;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid == 0) {
+    pub->flips = 0;
+    pub->fin = -1;
+  }
+  const long long pos0 = a.ctr->u_pos, log0 = a.ctr->log_len;
+  const int r = lane & 15;
+  const int cf = (int)a.conf[w0 + (r < Wn ? r : Wn - 1)];
+  window_block_staged<GT, FLV, 16>(a, Bn, St, Zw, Wn, tid, lane, wave);
+  if (wave == 3 && lane < 16) {                  // (waves 0 and 1 form the block)
+    double u = 1.0;
+    if (a.uniforms) {
+      if (pos0 + lane < a.n_uniforms) u = a.uniforms[pos0 + lane];
+    } else {
+      u = counter_uniform(a.seed, (unsigned long long)(pos0 + lane));
+    }
+    U[lane] = u;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    Win16Tally tl = {0, 0, 0, 0};
+    decide16<GT, FLV>(a, Bn, pub, U, 15, cf, w0, Wn, log0, lane, tl);
+    if (lane == 0) {
+      ChainCounters* c = a.ctr;
+      c->u_pos = pos0 + tl.used;
+      c->accepted += tl.flips;
+      c->proposed += Wn;
+      c->negative += tl.neg;
+      c->ties += tl.ties;
+      if (a.uniforms && pos0 + tl.used > a.n_uniforms) c->exhausted = 1;
+      c->log_len = log0 + Wn;
+      c->flushes += 1;
+    }
+  } else if (wave == 2) {
+    factor16<GT, FLV>(a, Bn, pub, Wn, lane, a.Y, a.S, nullptr);
+  }
+}
+
+// Workgroup 0 of a slice launch with 16-site windows (see window_slice_kernel).  The slice's
+// uniforms and field are brought to LDS once.  Per window, with two workgroup barriers:
+//   waves 0 and 1 form the block from LDS (prefetched operands, the previous window's factor),
+//   while wave 2 publishes the previous window's factor (its own stores);
+//   then wave 0 decides, wave 2 builds the factor, and wave 3 prefetches the next window's
+//   operands once every application of window k - 1 is done.
+template <typename GT, int FLV>
+__device__ __forceinline__ void slice16_role(const WindowSlice<GT>& s, unsigned char* smem, unsigned long long* ready,
+                                             const unsigned long long* applied, unsigned long long epoch,
+                                             unsigned long long done, unsigned long long* errc) {
+  static_assert(sizeof(GT) == 8, "one launch per slice: FP64");
+  constexpr int LD = 17, MAT = 16 * LD;
+  double* Bn = reinterpret_cast<double*>(smem);
+  GT* St = reinterpret_cast<GT*>(Bn + FLV * MAT);
+  GT* pf = St;                                   // [3 FLV][16][LD]
+  GT* yl = St + 3 * FLV * MAT;                   // [FLV][16][LD]
+  Win16Pub* pub = reinterpret_cast<Win16Pub*>(St + 4 * FLV * MAT);
+  double* U = reinterpret_cast<double*>(pub + 1);
+  int8_t* cl = reinterpret_cast<int8_t*>(U + s.a.n);
+  const int n = s.a.n, nw = s.nw;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15;
+  ChainCounters* ctr = s.a.ctr;
+  const long long pos0 = ctr->u_pos, log0 = ctr->log_len;
+  for (int i = tid; i < n; i += 256) {
+    double u = 1.0;
+    if (s.a.uniforms) {
+      if (pos0 + i < s.a.n_uniforms) u = s.a.uniforms[pos0 + i];
+    } else {
+      u = counter_uniform(s.a.seed, (unsigned long long)(pos0 + i));
+    }
+    U[i] = u;
+    cl[i] = s.a.conf[i];
+  }
+  Win16Tally tl = {0, 0, 0, 0};
+  for (int k = 0; k < nw; k++) {
+    const int w0 = k * 16, Wn = n - w0 < 16 ? n - w0 : 16;
+    if (tid == 0) {
+      pub->flips = 0;
+      pub->fin = -1;
+    }
+    if (wave == 2 && k > 0) {
+      // the previous window's factor and flip count are this wave's own stores
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      if (lane == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_store(ready + (k - 1), epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (k == 0) {                                // no flips yet: G[w, w] itself
+      for (int e = tid; e < FLV * 256; e += 256) {
+        const int b = e >> 8, c = (e >> 4) & 15, i = e & 15;
+        Bn[b * MAT + c * LD + i] = s.B[0][(size_t)b * n * n + (size_t)(c < Wn ? c : Wn - 1) * n + (i < Wn ? i : Wn - 1)];
+      }
+    } else if (wave < FLV) {
+      window_block_form<GT, FLV, 16>(Bn, pf, 3, yl, 1, pub->m > 0, nullptr, lane, wave);
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int kmax = n - 1 - tl.used;
+      decide16<GT, FLV>(s.a, Bn, pub, U + tl.used, kmax < 15 ? kmax : 15, (int)cl[w0 + (r < Wn ? r : Wn - 1)], w0, Wn,
+                        log0 + w0, lane, tl);
+    } else if (wave == 2) {
+      factor16<GT, FLV>(s.a, Bn, pub, Wn, lane, s.Y + (size_t)(k & 1) * FLV * 256, s.S + (k & 1) * 17, yl);
+    } else if (wave == 3 && k + 1 < nw) {
+      // G[w', w'], G[w', w], G[w, w'] of the next window w' from B[k % 2], which the updates of
+      // window k - 1 write
+      if (k > 0) {
+        long long polls = 0;
+        bool ok = true;
+        while (__hip_atomic_load(applied + (k - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < done) {
+          if (++polls > s.a.wait_limit) { ok = false; break; }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (!ok && lane == 0) atomicAdd(errc, 1ull);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      const int w0n = w0 + 16, Wnn = n - w0n < 16 ? n - w0n : 16;
+      const int rw = w0n + (r < Wnn ? r : Wnn - 1), rp = w0 + r;
+      GT v[3][FLV][4];
+#pragma unroll
+      for (int b = 0; b < FLV; b++) {
+        const GT* Gb = s.B[k & 1] + (size_t)b * n * n;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int c = (lane >> 4) + 4 * q;
+          const int cw = w0n + (c < Wnn ? c : Wnn - 1), cp = w0 + c;
+          v[0][b][q] = Gb[(size_t)rw + (size_t)cw * n];
+          v[1][b][q] = Gb[(size_t)rw + (size_t)cp * n];
+          v[2][b][q] = Gb[(size_t)rp + (size_t)cw * n];
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < FLV; b++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int mat = 0; mat < 3; mat++)
+            pf[(3 * b + mat) * MAT + ((lane >> 4) + 4 * q) * LD + r] = v[mat][b][q];
+    }
+    __syncthreads();
+  }
+  if (wave == 2) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    if (lane == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __hip_atomic_store(ready + (nw - 1), epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (tid == 0) {
+    ctr->u_pos = pos0 + tl.used;
+    ctr->accepted += tl.flips;
+    ctr->proposed += n;
+    ctr->negative += tl.neg;
+    ctr->ties += tl.ties;
+    if (s.a.uniforms && pos0 + tl.used > s.a.n_uniforms) ctr->exhausted = 1;
+    ctr->log_len = log0 + n;
+    ctr->flushes += nw;
+  }
+}
+
+// Gd_b = Gs_b - C_b (Y_b R_b) on a run of 64 x 64 tiles (down a column of tiles, then the next
+// column), for a window's flips with its dense factor Y over positions wp .. wp + W - 1:
+// C = (I - Gs)[:, wp:wp+W] and R = Gs[wp:wp+W, :] are contiguous strips of the source copy (the
+// update writes the other copy, so no tile changes what another still reads).  The rank-W
+// product is computed transposed, tile^T -= Z^T C^T, so accumulator element r of lane l is
+// G[r0 + l%16][c0 + row(l, r)]: quarter-waves touch 16 consecutive rows of a column.
 //
-// What bounds a tile is memory latency (the strips were just written by other workgroups), so
-// every operand is loaded straight into the matrix-core registers, all in flight at once: wave w
-// owns rows 16 w .. (C's operand) and columns 16 w .. of Z = Y R (R's).  Only Z goes through
-// LDS, formed once per column of tiles, and the next tile's loads are issued before this tile's
-// products.  Against operands staged through LDS in turn, one tile after the other: 4.0 -> 3.6 us
-// for the one tile per workgroup of n = 256, 23 -> 18.5 us for the four of n = 1024 with two
-// flavours (a sweep of 32x32 sites 230 -> 216 ms).
+// What bounds a tile is memory latency (the strips were just written by other workgroups) and,
+// with one wave per SIMD, the instruction stream.  So every operand is loaded straight into the
+// matrix-core registers, all in flight at once: wave w owns rows 16 w .. (C's operand) and
+// columns 16 w .. of Z = Y R (R's).  Only Z goes through LDS, formed once per column of tiles, and
+// the next tile's loads are issued before this tile's products.  Inside the lattice, addresses are
+// a uniform base and one lane offset.  The first tile's operands do not depend on Y: a slice
+// launch has them in registers before it waits for the factor (`ready`).
+struct TileRun {
+  int b, rt, ct, count;           // flavour block, row and column of the first tile; tiles
+};
+__device__ __forceinline__ TileRun tile_run(int t0, int t1, int n) {
+  const int nt = (n + 63) >> 6;
+  const int b = t0 / (nt * nt), rem = t0 - b * nt * nt;
+  return TileRun{b, rem % nt, rem / nt, t1 - t0};
+}
+
 template <typename GT, int W>
 struct ApplyTile {
   typename V4<GT>::type acc[4];   // the tile of Gs: rows 16 wave + li, columns 16 j + row(lane, r)
   GT cg[W / 4];                   // Gs[row][wp + 4 s + lk]
 };
 
+// Element `off` bytes after a uniform base (a 32-bit lane offset: 8 n^2 bytes at most).
+template <typename GT>
+__device__ __forceinline__ GT load_at(const GT* base, unsigned int off) {
+  return *reinterpret_cast<const GT*>(reinterpret_cast<const char*>(base) + off);
+}
+
 template <typename GT, int W>
 __device__ __forceinline__ void apply_load(ApplyTile<GT, W>& x, const GT* Gb, int n, int wp, int r0, int c0,
                                            int lane, int wave) {
-  const int li = lane & 15, lk = lane >> 4;
+  const int li = lane & 15, lk = lane >> 4, lc = mfma_row<GT>(lane, 0);
+  if (r0 + 64 <= n && c0 + 64 <= n && wp + W <= n) {
+    const unsigned int row = 16 * wave + li;
+    const unsigned int oc = (unsigned int)sizeof(GT) * (row + (unsigned int)lk * n);
+    const unsigned int oa = (unsigned int)sizeof(GT) * (row + (unsigned int)lc * n);
+#pragma unroll
+    for (int s = 0; s < W / 4; s++) x.cg[s] = load_at(Gb + r0 + (size_t)(wp + 4 * s) * n, oc);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) x.acc[j][r] = load_at(Gb + r0 + (size_t)(c0 + 16 * j + mfma_row<GT>(0, r)) * n, oa);
+    return;
+  }
   const int row = r0 + 16 * wave + li;
   const size_t rowc = (size_t)(row < n ? row : n - 1);
 #pragma unroll
@@ -1005,61 +1490,72 @@ __device__ __forceinline__ void apply_load(ApplyTile<GT, W>& x, const GT* Gb, in
     }
 }
 
+// R's operand of this wave's 16 columns of Z.
 template <typename GT, int W>
-__device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __restrict__ Gs,
-                                           const int* __restrict__ Sp, const GT* __restrict__ Y, int n,
-                                           int wp, int t0, int t1, unsigned char* smem) {
+__device__ __forceinline__ void apply_load_r(GT (&rv)[W / 4], const GT* Gb, int n, int wp, int c0, int lane, int wave) {
+  const int li = lane & 15, lk = lane >> 4;
+  if (c0 + 64 <= n && wp + W <= n) {
+    const unsigned int o = (unsigned int)sizeof(GT) * (lk + (unsigned int)(16 * wave + li) * n);
+#pragma unroll
+    for (int s = 0; s < W / 4; s++) rv[s] = load_at(Gb + wp + 4 * s + (size_t)c0 * n, o);
+    return;
+  }
+  const int zc = c0 + 16 * wave + li;
+#pragma unroll
+  for (int s = 0; s < W / 4; s++) {
+    const int k = wp + 4 * s + lk;
+    const GT v = Gb[(size_t)(k < n ? k : n - 1) + (size_t)(zc < n ? zc : n - 1) * n];
+    rv[s] = zc < n ? v : GT(0);
+  }
+}
+
+template <typename GT, int W, typename Ready>
+__device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __restrict__ Gs, const int* Sp,
+                                           const GT* Y, int n, int wp, TileRun t, unsigned char* smem, Ready ready) {
   typedef typename V4<GT>::type acc_t;
   constexpr int KS = W / 4, CT = W / 16;
   const int nt = (n + 63) >> 6;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lk = lane >> 4;
+  const size_t nn = (size_t)n * n;
   GT* Zs = reinterpret_cast<GT*>(smem);     // W x 65  [k][col]
-  const int m = Sp[0];
   ApplyTile<GT, W> cur, nxt;
-  {
-    const int b = t0 / (nt * nt), rem = t0 - b * nt * nt;
-    apply_load<GT, W>(cur, Gs + (size_t)b * n * n, n, wp, (rem % nt) * 64, (rem / nt) * 64, lane, wave);
-  }
-  int zcol = -1;                            // the column of tiles Zs holds (counted over the blocks)
-  for (int t = t0; t < t1; t++) {
-    const int b = t / (nt * nt), rem = t - b * nt * nt;
-    const int r0 = (rem % nt) * 64, c0 = (rem / nt) * 64;
-    const size_t off = (size_t)b * n * n;
-    const GT* Gb = Gs + off;
-    GT* Gw = Gd + off;
-    const bool newz = t / nt != zcol;
-    GT rv[KS], yv[CT][KS];
-    const int zc = c0 + 16 * wave + li;
+  GT rv[KS], yv[CT][KS];
+  apply_load<GT, W>(cur, Gs + t.b * nn, n, wp, t.rt * 64, t.ct * 64, lane, wave);
+  apply_load_r<GT, W>(rv, Gs + t.b * nn, n, wp, t.ct * 64, lane, wave);
+  ready();
+  const int m = Sp[0];
+  for (int i = 0; i < t.count; i++) {
+    const int r0 = t.rt * 64, c0 = t.ct * 64, b = t.b;
+    const bool newz = i == 0 || t.rt == 0;
     if (newz) {
+      if (i > 0) apply_load_r<GT, W>(rv, Gs + b * nn, n, wp, c0, lane, wave);
 #pragma unroll
-      for (int s = 0; s < KS; s++) {
-        const int k = wp + 4 * s + lk;
-        rv[s] = Gb[(size_t)(k < n ? k : n - 1) + (size_t)(zc < n ? zc : n - 1) * n];
+      for (int q = 0; q < CT; q++)
+#pragma unroll
+        for (int s = 0; s < KS; s++) yv[q][s] = Y[(size_t)b * W * W + (size_t)(16 * q + li) * W + 4 * s + lk];
+    }
+    if (++t.rt == nt) {
+      t.rt = 0;
+      if (++t.ct == nt) {
+        t.ct = 0;
+        t.b++;
       }
-#pragma unroll
-      for (int i = 0; i < CT; i++)
-#pragma unroll
-        for (int s = 0; s < KS; s++) yv[i][s] = Y[(size_t)b * W * W + (size_t)(16 * i + li) * W + 4 * s + lk];
     }
-    if (t + 1 < t1) {
-      const int b1 = (t + 1) / (nt * nt), rem1 = t + 1 - b1 * nt * nt;
-      apply_load<GT, W>(nxt, Gs + (size_t)b1 * n * n, n, wp, (rem1 % nt) * 64, (rem1 / nt) * 64, lane, wave);
-    }
+    if (i + 1 < t.count) apply_load<GT, W>(nxt, Gs + t.b * nn, n, wp, t.rt * 64, t.ct * 64, lane, wave);
     if (m > 0) {
       if (newz) {
-        if (zcol >= 0) __syncthreads();     // the waves have read the previous column's Z
+        if (i > 0) __syncthreads();         // the waves have read the previous column's Z
         // Z[:, 16 wave : 16 wave + 16] = Y R[:, same columns]
 #pragma unroll
-        for (int i = 0; i < CT; i++) {
+        for (int q = 0; q < CT; q++) {
           acc_t z = {0, 0, 0, 0};
 #pragma unroll
-          for (int s = 0; s < KS; s++) z = mfma16(yv[i][s], zc < n ? rv[s] : GT(0), z);
+          for (int s = 0; s < KS; s++) z = mfma16(yv[q][s], rv[s], z);
 #pragma unroll
-          for (int r = 0; r < 4; r++) Zs[(16 * i + mfma_row<GT>(lane, r)) * 65 + 16 * wave + li] = z[r];
+          for (int r = 0; r < 4; r++) Zs[(16 * q + mfma_row<GT>(lane, r)) * 65 + 16 * wave + li] = z[r];
         }
         __syncthreads();
-        zcol = t / nt;
       }
       const int row = r0 + 16 * wave + li;
 #pragma unroll
@@ -1070,15 +1566,27 @@ __device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __res
         for (int j = 0; j < 4; j++) cur.acc[j] = mfma16(-Zs[k * 65 + 16 * j + li], bv, cur.acc[j]);
       }
     }
-    const int grow = r0 + 16 * wave + li;
+    GT* Gw = Gd + b * nn;
+    if (r0 + 64 <= n && c0 + 64 <= n) {
+      const unsigned int o = (unsigned int)sizeof(GT) * (16 * wave + li + (unsigned int)mfma_row<GT>(lane, 0) * n);
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+      for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int gcol = c0 + 16 * j + mfma_row<GT>(lane, r);
-        if (grow < n && gcol < n) Gw[(size_t)grow + (size_t)gcol * n] = cur.acc[j][r];
-      }
-    cur = nxt;
+        for (int r = 0; r < 4; r++) {
+          GT* base = Gw + r0 + (size_t)(c0 + 16 * j + mfma_row<GT>(0, r)) * n;
+          *reinterpret_cast<GT*>(reinterpret_cast<char*>(base) + o) = cur.acc[j][r];
+        }
+    } else {
+      const int grow = r0 + 16 * wave + li;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int gcol = c0 + 16 * j + mfma_row<GT>(lane, r);
+          if (grow < n && gcol < n) Gw[(size_t)grow + (size_t)gcol * n] = cur.acc[j][r];
+        }
+    }
+    if (i + 1 < t.count) cur = nxt;
   }
 }
 
@@ -1089,11 +1597,12 @@ template <typename GT, int FLV, int W>
 __global__ __launch_bounds__(256) void window_kernel(WindowArgs<GT> a) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (blockIdx.x == 0) {
-    window_role<GT, FLV, W>(a, smem);
+    if constexpr (W == 16) window16_role<GT, FLV>(a, smem);
+    else window_role<GT, FLV, W>(a, smem);
     return;
   }
   const int t = (int)blockIdx.x - 1;
-  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, t, t + 1, smem);
+  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(t, t + 1, a.n), smem, []() {});
 }
 
 // The last window's application alone.
@@ -1101,7 +1610,7 @@ template <typename GT, int W>
 __global__ __launch_bounds__(256) void window_apply_kernel(WindowArgs<GT> a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int t = (int)blockIdx.x;
-  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, t, t + 1, smem);
+  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(t, t + 1, a.n), smem, []() {});
 }
 
 // Bounded wait until *p >= v (device scope); false when the bound is reached.
@@ -1114,11 +1623,12 @@ __device__ __forceinline__ bool wait_at_least(const unsigned long long* p, unsig
   return true;
 }
 
-// One launch per slice.  Workgroup 0 runs windows 0 .. nw - 1 back to back, as in
-// window_kernel, pipelined (SliceCtl): window k's block operands were prefetched during window
-// k - 1 once every application of window k - 2 was done (window k reads their output copy),
-// and window k - 1's factor is published once window k's block is formed.  Workgroup 1 + i applies window j to its
-// own run of tiles once window j is published and every application of window j - 1 is
+// One launch per slice.  Workgroup 0 runs windows 0 .. nw - 1 back to back, pipelined
+// (slice16_role; SliceCtl for 32 sites): window k's block operands were prefetched during window
+// k - 1 once every application of window k - 2 was done (window k reads their output copy), and
+// window k - 1's factor is published beside or right after window k's block.  Workgroup 1 + i
+// applies window j to its own run of tiles once window j is published and every application of
+// window j - 1 is
 // done (whose source copy window j's application overwrites).  Every wait is bounded; a wait
 // that gives up counts a device error and the launch still ends.  All workgroups are resident
 // at once (one per CU, 1 + napply <= 129), and a workgroup waits only for work that needs no
@@ -1136,48 +1646,44 @@ __global__ __launch_bounds__(256) void window_slice_kernel(WindowSlice<GT> s) {
   const size_t ysz = (size_t)FLV * W * W;
   const long long limit = s.a.wait_limit;
   if (blockIdx.x == 0) {
-    // window k's block operands: window 0's from global memory, every later window's
-    // prefetched during the previous window (from the copy that window k - 2's updates
-    // write, after they are done); window k - 1 is published once window k's block is formed
-    GT* pf = reinterpret_cast<GT*>(smem + window_lds<GT, FLV, W>());
-    SliceCtl<GT> sc;
-    sc.pf = pf;
-    sc.yl = pf + (size_t)3 * FLV * W * (W + 1);
-    sc.errc = errc;
-    sc.limit = limit;
-    for (int k = 0; k < s.nw; k++) {
-      __syncthreads();
-      WindowArgs<GT> a = s.a;
-      a.w0 = k * W;
-      a.wp = a.w0 - W;
-      a.do_window = 1;
-      a.G = k ? s.B[(k - 1) & 1] : s.B[0];
-      a.Gd = k ? s.B[k & 1] : s.B[1];
-      a.Sp = k ? s.S + ((k - 1) & 1) * (W + 1) : nullptr;
-      a.Yp = k ? s.Y + ((k - 1) & 1) * ysz : nullptr;
-      a.S = s.S + (k & 1) * (W + 1);
-      a.Y = s.Y + (k & 1) * ysz;
-      sc.pf_in = k > 0;
-      sc.gnext = k + 1 < s.nw ? s.B[k & 1] : nullptr;         // window k + 1 reads B[k % 2]
-      sc.wait_p = k >= 1 ? applied + (k - 1) : nullptr;
-      sc.wait_v = done;
-      // Where window k - 1 is published: short windows (W = 16) publish each window as soon
-      // as its stores have completed (the fourth wave issues the release while the next window
-      // starts), so that its updates are done before the fourth wave's next prefetch waits for
-      // them; longer windows publish once the next window's block is formed, which keeps the
-      // wait for the stores off their path (measured: 16 sites 71.5 -> 70.5 ms per sweep at
-      // n = 256, 32 sites 73.7 -> 74.8 ms with the early form).
-      constexpr bool kEarly = W <= 16;
-      sc.pub_p = !kEarly && k >= 1 ? ready + (k - 1) : nullptr;
-      sc.pub_v = e + 1;
-      window_role<GT, FLV, W>(a, smem, &sc);
-      if (kEarly || k + 1 == s.nw) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);     // this window's global stores have completed
+    if constexpr (W == 16) {
+      slice16_role<GT, FLV>(s, smem, ready, applied, e, done, errc);
+    } else {
+      // window k's block operands: window 0's from global memory, every later window's
+      // prefetched during the previous window (from the copy that window k - 2's updates
+      // write, after they are done); window k - 1 is published once window k's block is
+      // formed, which keeps the wait for its stores off the windows' path
+      GT* pf = reinterpret_cast<GT*>(smem + window_lds<GT, FLV, W>());
+      SliceCtl<GT> sc;
+      sc.pf = pf;
+      sc.yl = pf + (size_t)3 * FLV * W * (W + 1);
+      sc.errc = errc;
+      sc.limit = limit;
+      for (int k = 0; k < s.nw; k++) {
         __syncthreads();
-        if (tid == 192) {
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-          __hip_atomic_store(ready + k, e + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        WindowArgs<GT> a = s.a;
+        a.w0 = k * W;
+        a.wp = a.w0 - W;
+        a.do_window = 1;
+        a.G = k ? s.B[(k - 1) & 1] : s.B[0];
+        a.Gd = k ? s.B[k & 1] : s.B[1];
+        a.Sp = k ? s.S + ((k - 1) & 1) * (W + 1) : nullptr;
+        a.Yp = k ? s.Y + ((k - 1) & 1) * ysz : nullptr;
+        a.S = s.S + (k & 1) * (W + 1);
+        a.Y = s.Y + (k & 1) * ysz;
+        sc.pf_in = k > 0;
+        sc.gnext = k + 1 < s.nw ? s.B[k & 1] : nullptr;         // window k + 1 reads B[k % 2]
+        sc.wait_p = k >= 1 ? applied + (k - 1) : nullptr;
+        sc.wait_v = done;
+        sc.pub_p = k >= 1 ? ready + (k - 1) : nullptr;
+        sc.pub_v = e + 1;
+        window_role<GT, FLV, W>(a, smem, &sc);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);     // the last window's global stores have completed
+      __syncthreads();
+      if (tid == 192) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_store(ready + (s.nw - 1), e + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
     if (tid == 0) {
@@ -1190,17 +1696,21 @@ __global__ __launch_bounds__(256) void window_slice_kernel(WindowSlice<GT> s) {
   const int nt = (s.a.n + 63) >> 6;
   const int tiles = FLV * nt * nt, per = (tiles + s.napply - 1) / s.napply;
   const int t0 = ((int)blockIdx.x - 1) * per, t1 = t0 + per < tiles ? t0 + per : tiles;
-  for (int j = 0; j < s.nw; j++) {
+  const TileRun run = tile_run(t0, t1, s.a.n);
+  auto wait_for = [&](const unsigned long long* p, unsigned long long v) {
     if (tid == 0) {
-      bool ok = wait_at_least(ready + j, e + 1, limit);
-      if (ok && j >= 1) ok = wait_at_least(applied + (j - 1), done, limit);
-      if (!ok) atomicAdd(errc, 1ull);
+      if (!wait_at_least(p, v, limit)) atomicAdd(errc, 1ull);
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
-    if (t0 < t1)
+  };
+  for (int j = 0; j < s.nw; j++) {
+    if (j >= 1) wait_for(applied + (j - 1), done);
+    if (run.count > 0)
       apply_tiles<GT, W>(s.B[(j + 1) & 1], s.B[j & 1], s.S + (j & 1) * (W + 1), s.Y + (j & 1) * ysz, s.a.n,
-                         j * W, t0, t1, smem);
+                         j * W, run, smem, [&]() { wait_for(ready + j, e + 1); });
+    else
+      wait_for(ready + j, e + 1);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
     if (tid == 0) {
@@ -1226,12 +1736,15 @@ int window_size(int n, int flv) {
 }
 
 template <typename GT, int FLV, int W>
+constexpr size_t role_lds() { return W == 16 ? win16_lds<GT, FLV>(16) : window_lds<GT, FLV, W>(); }
+
+template <typename GT, int FLV, int W>
 static void launch_window_w(const WindowArgs<GT>& a, hipStream_t s) {
   const int nt = (a.n + 63) / 64;
   const int tiles = a.Yp ? FLV * nt * nt : 0;
   if (a.do_window) {
-    const size_t lds = tiles && apply_lds<GT, W>() > window_lds<GT, FLV, W>() ? apply_lds<GT, W>()
-                                                                           : window_lds<GT, FLV, W>();
+    const size_t lds = tiles && apply_lds<GT, W>() > role_lds<GT, FLV, W>() ? apply_lds<GT, W>()
+                                                                         : role_lds<GT, FLV, W>();
     hipLaunchKernelGGL((window_kernel<GT, FLV, W>), dim3(1 + tiles), dim3(256), lds, s, a);
   } else if (tiles) {
     hipLaunchKernelGGL((window_apply_kernel<GT, W>), dim3(tiles), dim3(256), (apply_lds<GT, W>()), s, a);
@@ -1248,8 +1761,13 @@ __global__ __launch_bounds__(256) void window_multi_kernel(const WindowArgs<GT>*
   const WindowArgs<GT>& a = items[blockIdx.y];
   if (blockIdx.x == 0) {
     if (a.do_window) {
-      if (a.flv == 1) window_role<GT, 1, W>(a, smem);
-      else window_role<GT, 2, W>(a, smem);
+      if constexpr (W == 16) {
+        if (a.flv == 1) window16_role<GT, 1>(a, smem);
+        else window16_role<GT, 2>(a, smem);
+      } else {
+        if (a.flv == 1) window_role<GT, 1, W>(a, smem);
+        else window_role<GT, 2, W>(a, smem);
+      }
     }
     return;
   }
@@ -1257,12 +1775,12 @@ __global__ __launch_bounds__(256) void window_multi_kernel(const WindowArgs<GT>*
   const int nt = (a.n + 63) / 64;
   const int tile = (int)blockIdx.x - 1;
   if (tile >= a.flv * nt * nt) return;
-  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile, tile + 1, smem);
+  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(tile, tile + 1, a.n), smem, []() {});
 }
 
 template <int W>
 constexpr size_t window_multi_lds() {
-  constexpr size_t w1 = window_lds<double, 1, W>(), w2 = window_lds<double, 2, W>(), ap = apply_lds<double, W>();
+  constexpr size_t w1 = role_lds<double, 1, W>(), w2 = role_lds<double, 2, W>(), ap = apply_lds<double, W>();
   return (w1 > w2 ? (w1 > ap ? w1 : ap) : (w2 > ap ? w2 : ap));
 }
 
@@ -1300,7 +1818,9 @@ hipError_t launch_window_f64(const WindowArgs<double>& a, hipStream_t s) { retur
 
 template <int FLV, int W>
 static void launch_slice_w(const WindowSlice<double>& s, hipStream_t st) {
-  const size_t wl = window_lds<double, FLV, W>() + slice_extra_lds<double, FLV, W>(), al = apply_lds<double, W>();
+  const size_t wl = W == 16 ? win16_lds<double, FLV>(s.a.n)
+                            : window_lds<double, FLV, W>() + slice_extra_lds<double, FLV, W>();
+  const size_t al = apply_lds<double, W>();
   static_assert(window_lds<double, FLV, W>() % 16 == 0, "prefetch area alignment");
   static_assert(window_lds<double, FLV, W>() + slice_extra_lds<double, FLV, W>() <= 160 * 1024, "LDS");
   hipLaunchKernelGGL((window_slice_kernel<double, FLV, W>), dim3(1 + s.napply), dim3(256), wl > al ? wl : al, st, s);
