@@ -58,7 +58,8 @@ typedef struct {
   int precision;    /* DQMC_PRECISION_*                                                     */
   int check_propagation_error; /* DQMCParameters.check_propagation_error                   */
   int delay_depth;  /* sites per local-update window: <= 16 -> 16, <= 32 -> 32, else 64;
-                       0 = automatic (32)                                              */
+                       0 = automatic (16 while an update of G has at most 128 tiles of
+                       64 x 64, else 32)                                               */
   int device;       /* HIP device ordinal                                                   */
   double mixed_tolerance; /* DQMC_PRECISION_MIXED: bound on max|G_wrapped - G_scratch| at each
                              stabilisation; 0 = 1e-6.  Ignored in FP64.                    */

@@ -9,16 +9,18 @@
 // the diagonal interaction matrices enter as row / inner / column scalings generated
 // straight from the Hirsch field column, so they never exist as separate arrays.
 //
-// Tile: 32 x 32 per 256-thread workgroup (many workgroups even at n = 256); each wave64
-// owns one 16x16 output tile as a v_mfma_f64_16x16x4f64 (FP64) or v_mfma_f32_16x16x4f32
-// (FP32) accumulator.  Operand layout of the 16x16x4 instructions (wave64, lane l):
+// Tile: 32 x 32 per workgroup of 16 waves or 64 x 64 per workgroup of 8: each quadrant of the
+// tile has four (or two) waves, each with v_mfma_f64_16x16x4f64 (FP64) or
+// v_mfma_f32_16x16x4f32 (FP32) accumulators over their part of K, added through LDS at the end.
+// The waves of a SIMD share the loads and hide each other's latencies, where one wave per SIMD was
+// bound by its own instruction stream.  Operand layout of the 16x16x4 instructions (wave64, lane l):
 //   A (16 x 4): lane l supplies A[l % 16][l / 16]
 //   B (4 x 16): lane l supplies B[l / 16][l % 16]
 //   D (16 x 16): lane l holds D[row][l % 16], r = 0..3, with row = l / 16 + 4 r (FP64)
 //                or 4 (l / 16) + r (FP32); see mfma_row in common.h
-// K is staged through LDS in chunks of 128 with two buffers: a chunk's global loads are
-// all issued at once and the next chunk's loads are in flight during the current chunk's
-// products, so a product of K <= 256 costs about one memory round trip.
+// K is staged through LDS in chunks with two buffers: a chunk's global loads are all issued at
+// once and the next chunk's loads are in flight during the current chunk's products, so a
+// 32 x 32 tile with K <= 256 costs about one memory round trip.
 #include "common.h"
 
 namespace dqmc {
@@ -38,19 +40,27 @@ __device__ __forceinline__ fx4 mfma16(float a, float b, fx4 c) {
 }
 
 // Tile geometry: TILE x TILE outputs per workgroup, K staged in chunks of KC.  TILE = 32
-// (each wave one 16x16 accumulator, KC = 128) for launches with few tiles; TILE = 64 (each
-// wave a 32x32 quadrant as 2 x 2 accumulators, KC = 64) for launches with many, where it
-// halves the operand traffic per flop.  Every output element accumulates its k-steps of 4
-// in the same order with either geometry, so the two give identical results.
+// (a wave: one 16x16 fragment) where a launch has few tiles, TILE = 64 (a wave: a 32x32 quadrant
+// as 2 x 2 fragments) where it has many: half the operand traffic per flop.  With either, an
+// element is the sum (p0 + p1) + (p2 + p3) of four accumulators, p_q over the pieces
+// k = 16 (4 i + q) .. + 15, i = 0, 1, ..., in order, so the two give identical results: a wave of
+// the 32-wide tile holds one of the four, a wave of the 64-wide tile two.
 template <int TILE> struct TileCfg {
+  static constexpr int Threads = TILE == 32 ? 1024 : 512;
+  static constexpr int Groups = Threads / 256;            // waves per quadrant
+  static constexpr int Parts = 4 / Groups;                // accumulators per wave and fragment
   static constexpr int KC = TILE == 32 ? 128 : 64;
   static constexpr int LD = TILE + 1;
   static constexpr int F = TILE / 32;                     // 16x16 fragments per wave and side
-  static constexpr int LPT = 2 * TILE * KC / 256;         // loads per thread per chunk (32)
+  static constexpr int LPT = 2 * TILE * KC / Threads;     // loads per thread per chunk (8, 16)
 };
 
 template <typename T, int TILE>
-constexpr size_t gemm_lds_bytes() { return sizeof(T) * 2 * 2 * TileCfg<TILE>::KC * TileCfg<TILE>::LD; }
+constexpr size_t gemm_lds_bytes() {
+  const size_t stage = sizeof(T) * 2 * 2 * TileCfg<TILE>::KC * TileCfg<TILE>::LD;
+  const size_t sums = sizeof(T) * 16 * TileCfg<TILE>::F * TileCfg<TILE>::F * 16 * 17;
+  return stage > sums ? stage : sums;
+}
 
 // XCD-aware tile order.  Workgroups go to the 8 XCDs round-robin by linear id, and each XCD
 // has its own L2: with the plain order, XCD k gets the tiles of row block k, so every XCD
@@ -78,11 +88,12 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by, int& bz) {
 // the kernel arguments (a separate instantiation, so the one-chain path reads its items
 // straight from the argument segment)
 template <typename T, int TA, int TB, bool TAB, int TILE>
-__global__ __launch_bounds__(256) void gemm_kernel(GemmBatch<T> batch) {
+__global__ __launch_bounds__(TileCfg<TILE>::Threads) void gemm_kernel(GemmBatch<T> batch) {
   typedef typename AccT<T>::type acc_t;
   constexpr int kTM = TILE, kTN = TILE, kKC = TileCfg<TILE>::KC, kLD = TileCfg<TILE>::LD;
   constexpr int kF = TileCfg<TILE>::F, kLoadsPerThread = TileCfg<TILE>::LPT;
   constexpr int kHalf = kLoadsPerThread / 2;
+  constexpr int kThreads = TileCfg<TILE>::Threads, kGroups = TileCfg<TILE>::Groups, kParts = TileCfg<TILE>::Parts;
   int bx, by, bz;
   xcd_tile(bx, by, bz);
   const GemmItem<T>& it = TAB ? batch.items[bz] : batch.it[bz];
@@ -95,41 +106,43 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmBatch<T> batch) {
   T* Bs = As + 2 * kKC * kLD;                      // [2][kKC][kLD]  Bs[k][n]
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * (16 * kF), wn = (wave >> 1) * (16 * kF);
+  const int quad = wave & 3, kq = wave >> 2;       // quadrant of the tile, first piece of K
+  const int wm = (quad & 1) * (16 * kF), wn = (quad >> 1) * (16 * kF);
   const T* __restrict__ A = it.A;
   const T* __restrict__ B = it.B;
   const int lda = it.lda, ldb = it.ldb;
   const bool has_mid = diag_active(it.dmid);
   const int nch = (K + kKC - 1) / kKC;
 
-  // element q of this thread in a chunk: q < 16 -> A, else B; index e = tid + 256 (q % 16)
+  // element q of this thread in a chunk: q < kHalf -> A, else B; index e = tid + kThreads (q % kHalf)
   auto coord = [&](int q, int& mn, int& kk) {
-    const int e = tid + 256 * (q % kHalf);
+    const int e = tid + kThreads * (q % kHalf);
     const bool isA = q < kHalf;
     const bool kfast = isA ? TA == 1 : TB == 0;    // consecutive threads along k in memory
     if (kfast) { kk = e % kKC; mn = e / kKC; }
     else { mn = e % kTM; kk = e / kTM; }
   };
-  // two register sets (chunks of even / odd index), so that two chunks can be in flight
-  T ra[kLoadsPerThread], rb[kLoadsPerThread];
   // A chunk's loads are all issued before any is used: in-range (clamped) addresses, then
   // the out-of-range elements zeroed; the middle diagonal (a uniform choice per launch) is
   // gathered for the chunk's k values in a second batch of loads.
   auto load = [&](int c, T* reg) {
     const int k0 = c * kKC;
+    const int kl = K - 1 - k0, ml = M - 1 - m0, nl = N - 1 - n0;   // last in-range offsets
+    const T* Ac = TA == 0 ? A + m0 + (size_t)k0 * lda : A + k0 + (size_t)m0 * lda;
+    const T* Bc = TB == 0 ? B + k0 + (size_t)n0 * ldb : B + n0 + (size_t)k0 * ldb;
 #pragma unroll
     for (int q = 0; q < kLoadsPerThread; q++) {
       int mn, kk;
       coord(q, mn, kk);
-      const int gk = k0 + kk;
-      const int gkc = gk < K ? gk : K - 1;
-      if (q < kHalf) {
-        const int gm = m0 + mn, gmc = gm < M ? gm : M - 1;
-        reg[q] = TA == 0 ? A[(size_t)gmc + (size_t)gkc * lda] : A[(size_t)gkc + (size_t)gmc * lda];
-      } else {
-        const int gn = n0 + mn, gnc = gn < N ? gn : N - 1;
-        reg[q] = TB == 0 ? B[(size_t)gkc + (size_t)gnc * ldb] : B[(size_t)gnc + (size_t)gkc * ldb];
-      }
+      const bool isA = q < kHalf;
+      const int last = isA ? ml : nl;
+      mn = mn < last ? mn : last;
+      kk = kk < kl ? kk : kl;
+      // a uniform base and a 32-bit lane offset inside the chunk
+      const bool kfast = isA ? TA == 1 : TB == 0;
+      const unsigned int ld = isA ? lda : ldb;
+      const unsigned int off = (unsigned int)sizeof(T) * (kfast ? kk + mn * ld : mn + kk * ld);
+      reg[q] = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(isA ? Ac : Bc) + off);
     }
     if (has_mid) {
       double f[kHalf];
@@ -163,13 +176,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmBatch<T> batch) {
 #pragma unroll
       for (int q = 0; q < kHalf; q++) reg[q] = T(reg[q] * f[q]);
     }
+    if (m0 + kTM > M || n0 + kTN > N || k0 + kKC > K) {
 #pragma unroll
-    for (int q = 0; q < kLoadsPerThread; q++) {
-      int mn, kk;
-      coord(q, mn, kk);
-      const int gk = k0 + kk;
-      const bool ok = q < kHalf ? (m0 + mn < M && gk < K) : (n0 + mn < N && gk < K);
-      reg[q] = ok ? reg[q] : T(0);
+      for (int q = 0; q < kLoadsPerThread; q++) {
+        int mn, kk;
+        coord(q, mn, kk);
+        const int gk = k0 + kk;
+        const bool ok = q < kHalf ? (m0 + mn < M && gk < K) : (n0 + mn < N && gk < K);
+        reg[q] = ok ? reg[q] : T(0);
+      }
     }
   };
   auto store = [&](int buf, const T* reg) {
@@ -183,13 +198,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmBatch<T> batch) {
       else Bb[kk * kLD + mn] = reg[q];
     }
   };
-  acc_t acc[kF][kF];
+  acc_t acc[kParts][kF][kF];
 #pragma unroll
-  for (int i = 0; i < kF; i++)
+  for (int h = 0; h < kParts; h++)
 #pragma unroll
-    for (int j = 0; j < kF; j++) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int i = 0; i < kF; i++)
+#pragma unroll
+      for (int j = 0; j < kF; j++) acc[h][i][j] = acc_t{0, 0, 0, 0};
   const int li = lane & 15, lk = lane >> 4;
-  auto step = [&](const T* Ab, const T* Bb, int kk) {
+  auto step = [&](const T* Ab, const T* Bb, int kk, int h) {
     T av[kF], bv[kF];
 #pragma unroll
     for (int i = 0; i < kF; i++) av[i] = Ab[(kk + lk) * kLD + wm + 16 * i + li];
@@ -198,75 +215,118 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmBatch<T> batch) {
 #pragma unroll
     for (int i = 0; i < kF; i++)
 #pragma unroll
-      for (int j = 0; j < kF; j++) acc[i][j] = mfma16(av[i], bv[j], acc[i][j]);
+      for (int j = 0; j < kF; j++) acc[h][i][j] = mfma16(av[i], bv[j], acc[h][i][j]);
   };
   auto compute = [&](int c, int buf) {
     const T* Ab = As + buf * kKC * kLD;
     const T* Bb = Bs + buf * kKC * kLD;
     const int kend = K - c * kKC < kKC ? K - c * kKC : kKC;
-    if (kend == kKC) {
-      // a whole chunk: straight-line k-steps, so the LDS reads run ahead of the products
+    // (a whole chunk: straight-line k-steps, so the LDS reads run ahead of the products)
+    const bool whole = kend == kKC;
 #pragma unroll
-      for (int kk = 0; kk < kKC; kk += 4) step(Ab, Bb, kk);
-    } else {
-#pragma unroll 8
-      for (int kk = 0; kk < kKC; kk += 4)
-        if (kk < kend) step(Ab, Bb, kk);
-    }
+    for (int p = 0; p < kKC; p += 64)
+#pragma unroll
+      for (int h = 0; h < kParts; h++) {
+        const int k0 = p + 16 * (kq + kGroups * h);
+        if (whole || k0 + 16 <= kend) {
+#pragma unroll
+          for (int kk = 0; kk < 16; kk += 4) step(Ab, Bb, k0 + kk, h);
+        } else {
+#pragma unroll
+          for (int kk = 0; kk < 16; kk += 4)
+            if (k0 + kk < kend) step(Ab, Bb, k0 + kk, h);
+        }
+      }
   };
 
-  // chunk c lives in buffer c % 2 and arrives in register set ra (even c) or rb (odd c)
-  load(0, ra);
-  if (nch > 1) load(1, rb);
-  store(0, ra);
-  __syncthreads();
-  for (int c = 0; c < nch; c += 2) {
-    if (c + 2 < nch) load(c + 2, ra);
-    compute(c, 0);
-    if (c + 1 < nch) store(1, rb);
+  if constexpr (TILE == 32) {
+    // chunk c lives in buffer c % 2 and arrives in register set ra (even c) or rb (odd c), so
+    // that two chunks are in flight
+    T ra[kLoadsPerThread], rb[kLoadsPerThread];
+    load(0, ra);
+    if (nch > 1) load(1, rb);
+    store(0, ra);
     __syncthreads();
-    if (c + 1 < nch) {
-      if (c + 3 < nch) load(c + 3, rb);
-      compute(c + 1, 1);
-      if (c + 2 < nch) store(0, ra);
+    for (int c = 0; c < nch; c += 2) {
+      if (c + 2 < nch) load(c + 2, ra);
+      compute(c, 0);
+      if (c + 1 < nch) store(1, rb);
+      __syncthreads();
+      if (c + 1 < nch) {
+        if (c + 3 < nch) load(c + 3, rb);
+        compute(c + 1, 1);
+        if (c + 2 < nch) store(0, ra);
+        __syncthreads();
+      }
+    }
+  } else {
+    // one chunk ahead: its loads take no longer than a chunk's products
+    T ra[kLoadsPerThread];
+    load(0, ra);
+    store(0, ra);
+    __syncthreads();
+    for (int c = 0; c < nch; c++) {
+      if (c + 1 < nch) load(c + 1, ra);
+      compute(c, c & 1);
+      if (c + 1 < nch) store((c + 1) & 1, ra);
       __syncthreads();
     }
   }
+
+  // the four partial sums of every element through LDS (free after the last barrier): fragment
+  // (piece, quadrant, i, j) at 272 elements each, column by column with leading dimension 17
+  T* red = reinterpret_cast<T*>(smem);
+  constexpr int kFrag = 16 * 17, kQuarter = 4 * kF * kF * kFrag;
+#pragma unroll
+  for (int h = 0; h < kParts; h++)
+#pragma unroll
+    for (int i = 0; i < kF; i++)
+#pragma unroll
+      for (int j = 0; j < kF; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          red[(kq + kGroups * h) * kQuarter + ((quad * kF + i) * kF + j) * kFrag + li * 17 + mfma_row<T>(lane, r)] =
+              acc[h][i][j][r];
+  __syncthreads();
 
   const T alpha = T(batch.alpha), beta = T(batch.beta);
   const bool has_l = diag_active(it.dl), has_r = diag_active(it.dr), has_add = diag_active(it.dadd);
   T* __restrict__ Cm = it.C;
   const int ldc = it.ldc;
 #pragma unroll
-  for (int j = 0; j < kF; j++) {
-    const int col = n0 + wn + 16 * j + (lane & 15);
-    if (col >= N) continue;
-    const T sr = has_r ? T(diag_at(it.dr, col)) : T(1);
-#pragma unroll
-    for (int i = 0; i < kF; i++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = m0 + wm + 16 * i + mfma_row<T>(lane, r);
-        if (row >= M) continue;
-        T v = alpha * acc[i][j][r];
-        if (has_l) v *= T(diag_at(it.dl, row));
-        if (has_r) v *= sr;
-        T* dst = Cm + (size_t)row + (size_t)col * ldc;
-        if (beta != T(0)) v += beta * (*dst);
-        if (has_add && row == col) v += T(diag_at(it.dadd, row));
-        *dst = v;
-      }
-    }
+  for (int q = 0; q < TILE * TILE / kThreads; q++) {
+    // consecutive threads write consecutive rows of a column
+    const int e = tid + kThreads * q;
+    const int rt = e % TILE, ct = e / TILE;
+    const int row = m0 + rt, col = n0 + ct;
+    if (row >= M || col >= N) continue;
+    const int qd = rt / (16 * kF) + 2 * (ct / (16 * kF)), i = rt / 16 % kF, j = ct / 16 % kF;
+    const T* x = red + ((qd * kF + i) * kF + j) * kFrag + (ct & 15) * 17 + (rt & 15);
+    T v = alpha * ((x[0] + x[kQuarter]) + (x[2 * kQuarter] + x[3 * kQuarter]));
+    if (has_l) v *= T(diag_at(it.dl, row));
+    if (has_r) v *= T(diag_at(it.dr, col));
+    T* dst = Cm + (size_t)row + (size_t)col * ldc;
+    if (beta != T(0)) v += beta * (*dst);
+    if (has_add && row == col) v += T(diag_at(it.dadd, row));
+    *dst = v;
   }
 }
 
-// 64-wide tiles once a launch has at least 8 workgroups of 32 x 32 per CU to spread
-constexpr int64_t kWideTileMin = 8 * 256;
+// Which tile: one workgroup per CU at a time (LDS), so a launch lasts its rounds of 256 workgroups.
+// A round costs the tile's products (K / 4 steps of 64 clocks on every SIMD for TILE = 32, four
+// times that for 64) and its fill, sums and stores, about 6000 clocks (32) or 12000 (64).
+constexpr int64_t kGemmCUs = 256;
+static bool wide_tiles(int64_t t32, int64_t t64, int K) {
+  const int64_t step = (int64_t)((K + 3) / 4) * 64;
+  const int64_t c32 = (t32 + kGemmCUs - 1) / kGemmCUs * (step + 6000);
+  const int64_t c64 = (t64 + kGemmCUs - 1) / kGemmCUs * (4 * step + 12000);
+  return c64 < c32;
+}
 
 template <typename T, int TILE>
 static void launch_gemm_tile(const GemmBatch<T>& b, int Mx, int Nx, hipStream_t s) {
   dim3 grid((Mx + TILE - 1) / TILE, (Nx + TILE - 1) / TILE, b.count);
-  dim3 block(256);
+  dim3 block(TileCfg<TILE>::Threads);
   const size_t lds = gemm_lds_bytes<T, TILE>();
   const int sel = b.transA * 2 + b.transB;
   if (b.items) {
@@ -289,22 +349,25 @@ static void launch_gemm_tile(const GemmBatch<T>& b, int Mx, int Nx, hipStream_t 
 template <typename T>
 static hipError_t launch_gemm_t(const GemmBatch<T>& b, hipStream_t s) {
   if (b.count <= 0) return hipSuccess;
-  int Mx = 0, Nx = 0;
+  int Mx = 0, Nx = 0, Kx = 0;
   if (b.items) {
     // item table in device memory (checked by the host code that packed it)
     if (b.max_m < 1 || b.max_n < 1 || b.count > 65535) return hipErrorInvalidValue;
     Mx = b.max_m;
     Nx = b.max_n;
+    Kx = Mx;                       // (square products)
   } else {
     if (b.count > kMaxGemmItems) return hipErrorInvalidValue;
     for (int i = 0; i < b.count; i++) {
       if (b.it[i].K < 1) return hipErrorInvalidValue;
       if (b.it[i].M > Mx) Mx = b.it[i].M;
       if (b.it[i].N > Nx) Nx = b.it[i].N;
+      if (b.it[i].K > Kx) Kx = b.it[i].K;
     }
   }
-  const int64_t tiles32 = (int64_t)((Mx + 31) / 32) * ((Nx + 31) / 32) * b.count;
-  if (Mx >= 64 && Nx >= 64 && tiles32 >= kWideTileMin) launch_gemm_tile<T, 64>(b, Mx, Nx, s);
+  const int64_t t32 = (int64_t)((Mx + 31) / 32) * ((Nx + 31) / 32) * b.count;
+  const int64_t t64 = (int64_t)((Mx + 63) / 64) * ((Nx + 63) / 64) * b.count;
+  if (wide_tiles(t32, t64, Kx)) launch_gemm_tile<T, 64>(b, Mx, Nx, s);
   else launch_gemm_tile<T, 32>(b, Mx, Nx, s);
   return hipGetLastError();
 }

@@ -974,6 +974,22 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
   }
 }
 
+// A store that other workgroups read behind a flag in the same launch: written through to where
+// every XCD sees it (agent scope), so that its writer waits for the stores alone before it sets
+// the flag, and no write-back of the whole L2 stands between (application at n = 256: 0.95 -> 0.36
+// us from its last store to the flag; n = 1024, two flavours: slice launch 982 -> 890 us).
+template <bool SHARED, typename GT>
+__device__ __forceinline__ void put(GT* p, GT v) {
+  if constexpr (SHARED) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = v;
+}
+// This wave's stores have arrived (vmcnt(0)); no store moves past it.
+__device__ __forceinline__ void stores_done() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+}
+
 // ---------------------------------------------------------------------------------------
 // Windows of 16 sites.  One wave runs the decisions, a second builds the factor beside it, and
 // neither moves a row or a column of the block through LDS:
@@ -1086,10 +1102,12 @@ struct Win16Pub {
   int site[16];
   int flips, fin;        // flips published; final count (-1 while deciding)
   int m, pad;            // the last finished window's flips
+  // slices: windows whose factor is in LDS; the last window whose operands are; blocks formed
+  int factored, fetched, formed, pad2;
 };
 template <typename GT, int FLV>
 constexpr size_t win16_lds(int nu) {
-  return (size_t)FLV * 16 * 17 * 8 + (size_t)4 * FLV * 16 * 17 * sizeof(GT) +
+  return (size_t)FLV * 16 * 17 * 8 + (size_t)5 * FLV * 16 * 17 * sizeof(GT) +
          (sizeof(GT) == 4 ? (size_t)4 * 16 * 17 * 4 : 0) + sizeof(Win16Pub) + (size_t)nu * 9 + 16;
 }
 
@@ -1179,6 +1197,7 @@ __device__ __forceinline__ void decide16(const WindowArgs<GT>& a, const double* 
     if (lane == 0) pub->site[m] = t;
     m++;
   }
+  if (lane == 0) pub->m = m;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (lane == 0) {
     __hip_atomic_store(&pub->flips, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1191,7 +1210,6 @@ __device__ __forceinline__ void decide16(const WindowArgs<GT>& a, const double* 
   tl.ties += __popc((unsigned int)__ballot(tie) & win);
   tl.used += used;
   tl.flips += m;
-  if (lane == 0) pub->m = m;
   if (lane < Wn) {
     const bool acc = ((accepted >> lane) & 1u) != 0;
     if (a.dec_log && log0 + lane < a.log_cap) {
@@ -1202,12 +1220,12 @@ __device__ __forceinline__ void decide16(const WindowArgs<GT>& a, const double* 
   }
 }
 
-// The factor of one window (one wave, beside decide16): Y to global memory and, for slices, to LDS
-// (yl, leading dimension 17), the flip count to S.  The wait for a flip is bounded; giving up
-// leaves Y wrong, so it is counted as a device error that the host reports.
+// The factor of one window (one wave, beside decide16): to Y, row by row with leading dimension
+// ld.  Returns the flip count.  The wait for a flip is bounded; giving up leaves the factor wrong,
+// so it is counted as a device error that the host reports.
 template <typename GT, int FLV>
-__device__ __forceinline__ void factor16(const WindowArgs<GT>& a, const double* Bn, Win16Pub* pub, int Wn, int lane,
-                                         GT* Y, int* S, GT* yl) {
+__device__ __forceinline__ int factor16(const WindowArgs<GT>& a, const double* Bn, Win16Pub* pub, int Wn, int lane,
+                                        GT* Y, int ld) {
   const int f = lane >> 5, fb = FLV > 1 ? f : 0, r = lane & 15;
   const bool odd = (lane & 16) != 0;
   const double* Bf = Bn + (size_t)fb * 16 * 17;
@@ -1243,16 +1261,11 @@ __device__ __forceinline__ void factor16(const WindowArgs<GT>& a, const double* 
     k++;
   }
   if (odd && f < FLV) {
-    GT* Yr = Y + (size_t)f * 256 + r * 16;
+    GT* Yr = Y + (f * 16 + r) * ld;
 #pragma unroll
     for (int c = 0; c < 16; c++) Yr[c] = (GT)y[c];
-    if (yl) {
-      GT* yr = yl + (size_t)f * 16 * 17 + r * 17;
-#pragma unroll
-      for (int c = 0; c < 16; c++) yr[c] = (GT)y[c];
-    }
   }
-  if (lane == 0) S[0] = k;
+  return k;
 }
 
 // One 16-site window of one launch (window_kernel, window_multi_kernel): the block from the source
@@ -1299,16 +1312,34 @@ __device__ __forceinline__ void window16_role(const WindowArgs<GT>& a, unsigned 
       c->flushes += 1;
     }
   } else if (wave == 2) {
-    factor16<GT, FLV>(a, Bn, pub, Wn, lane, a.Y, a.S, nullptr);
+    const int m = factor16<GT, FLV>(a, Bn, pub, Wn, lane, a.Y, 16);
+    if (lane == 0) a.S[0] = m;
   }
 }
 
+// Wait for another wave of this workgroup, which reaches the count on its own (its waits for other
+// workgroups are bounded).
+__device__ __forceinline__ void wait_count(const int* p, int v) {
+  while (__hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < v) {}
+}
+__device__ __forceinline__ void set_count(int* p, int v, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (lane == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // Workgroup 0 of a slice launch with 16-site windows (see window_slice_kernel).  The slice's
-// uniforms and field are brought to LDS once.  Per window, with two workgroup barriers:
-//   waves 0 and 1 form the block from LDS (prefetched operands, the previous window's factor),
-//   while wave 2 publishes the previous window's factor (its own stores);
-//   then wave 0 decides, wave 2 builds the factor, and wave 3 prefetches the next window's
-//   operands once every application of window k - 1 is done.
+// uniforms and field are brought to LDS once; then the waves meet through counters in LDS:
+//   wave 0, and for a second flavour block window k's factor wave, form window k's block from LDS,
+//   once window k - 1's factor and the prefetched operands are there;
+//   wave 0 decides while window k's factor wave builds the factor, and that one then publishes it
+//   on its own: waves 1 and 2 take the windows in turn, so that one waits for its stores while the
+//   next window runs;
+//   wave 3 prefetches window k + 1's operands once window k's block is formed and every
+//   application of window k - 1 is done.
+// (Two barriers per window instead make every wave wait for the slowest one: 52.3 against 51.3 ms
+// per sweep of 16x16 sites.)  Per window of n = 256 the block takes 0.6 us, the decisions 4.1 (11
+// flips) and the factor's last flip 0.6; the loop that bounds it is publication, application (2.9
+// us) and prefetch.
 template <typename GT, int FLV>
 __device__ __forceinline__ void slice16_role(const WindowSlice<GT>& s, unsigned char* smem, unsigned long long* ready,
                                              const unsigned long long* applied, unsigned long long epoch,
@@ -1318,8 +1349,8 @@ __device__ __forceinline__ void slice16_role(const WindowSlice<GT>& s, unsigned 
   double* Bn = reinterpret_cast<double*>(smem);
   GT* St = reinterpret_cast<GT*>(Bn + FLV * MAT);
   GT* pf = St;                                   // [3 FLV][16][LD]
-  GT* yl = St + 3 * FLV * MAT;                   // [FLV][16][LD]
-  Win16Pub* pub = reinterpret_cast<Win16Pub*>(St + 4 * FLV * MAT);
+  GT* yl = St + 3 * FLV * MAT;                   // [2][FLV][16][LD]: factors of even and odd windows
+  Win16Pub* pub = reinterpret_cast<Win16Pub*>(St + 5 * FLV * MAT);
   double* U = reinterpret_cast<double*>(pub + 1);
   int8_t* cl = reinterpret_cast<int8_t*>(U + s.a.n);
   const int n = s.a.n, nw = s.nw;
@@ -1336,42 +1367,59 @@ __device__ __forceinline__ void slice16_role(const WindowSlice<GT>& s, unsigned 
     U[i] = u;
     cl[i] = s.a.conf[i];
   }
+  const int Wn0 = n < 16 ? n : 16;
+  for (int e = tid; e < FLV * 256; e += 256) {   // window 0: no flips yet, G[w, w] itself
+    const int b = e >> 8, c = (e >> 4) & 15, i = e & 15;
+    Bn[b * MAT + c * LD + i] = s.B[0][(size_t)b * n * n + (size_t)(c < Wn0 ? c : Wn0 - 1) * n + (i < Wn0 ? i : Wn0 - 1)];
+  }
+  if (tid == 0) {
+    pub->flips = 0;
+    pub->fin = -1;
+    pub->factored = pub->fetched = pub->formed = 0;
+  }
+  __syncthreads();
   Win16Tally tl = {0, 0, 0, 0};
   for (int k = 0; k < nw; k++) {
     const int w0 = k * 16, Wn = n - w0 < 16 ? n - w0 : 16;
-    if (tid == 0) {
-      pub->flips = 0;
-      pub->fin = -1;
-    }
-    if (wave == 2 && k > 0) {
-      // the previous window's factor and flip count are this wave's own stores
-      __builtin_amdgcn_s_waitcnt(0x0F70);
-      if (lane == 0) {
+    const int fw = 1 + (k & 1);                  // this window's factor wave
+    if (wave == 3 - fw) continue;                // (the other one publishes the previous window)
+    if (wave != 3) {
+      if (k > 0 && (wave == 0 || FLV > 1)) {
+        wait_count(&pub->factored, k);
+        wait_count(&pub->fetched, k);
+        if (tid == 0) {
+          pub->flips = 0;
+          pub->fin = -1;
+        }
+        const int b = wave == 0 ? 0 : 1;
+        window_block_form<GT, 1, 16>(Bn + b * MAT, pf + 3 * b * MAT, 3, yl + (((k - 1) & 1) * FLV + b) * MAT, 1, pub->m > 0, nullptr, lane, 0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0) __hip_atomic_fetch_add(&pub->formed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      wait_count(&pub->formed, FLV * k);
+      if (wave == 0) {
+        const int kmax = n - 1 - tl.used;
+        decide16<GT, FLV>(s.a, Bn, pub, U + tl.used, kmax < 15 ? kmax : 15, (int)cl[w0 + (r < Wn ? r : Wn - 1)], w0, Wn,
+                          log0 + w0, lane, tl);
+      } else {
+        GT* yk = yl + (k & 1) * FLV * MAT;
+        const int m = factor16<GT, FLV>(s.a, Bn, pub, Wn, lane, yk, LD);
+        set_count(&pub->factored, k + 1, lane);
+        // to global memory in whole lines
+        GT* Yk = s.Y + (size_t)(k & 1) * FLV * 256;
+#pragma unroll
+        for (int q = 0; q < FLV * 4; q++) Yk[64 * q + lane] = yk[(4 * q + (lane >> 4)) * LD + r];
+        if (lane == 0) s.S[(k & 1) * 17] = m;
+        stores_done();
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __hip_atomic_store(ready + (k - 1), epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_store(ready + k, epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-    }
-    if (k == 0) {                                // no flips yet: G[w, w] itself
-      for (int e = tid; e < FLV * 256; e += 256) {
-        const int b = e >> 8, c = (e >> 4) & 15, i = e & 15;
-        Bn[b * MAT + c * LD + i] = s.B[0][(size_t)b * n * n + (size_t)(c < Wn ? c : Wn - 1) * n + (i < Wn ? i : Wn - 1)];
-      }
-    } else if (wave < FLV) {
-      window_block_form<GT, FLV, 16>(Bn, pf, 3, yl, 1, pub->m > 0, nullptr, lane, wave);
-    }
-    __syncthreads();
-    if (wave == 0) {
-      const int kmax = n - 1 - tl.used;
-      decide16<GT, FLV>(s.a, Bn, pub, U + tl.used, kmax < 15 ? kmax : 15, (int)cl[w0 + (r < Wn ? r : Wn - 1)], w0, Wn,
-                        log0 + w0, lane, tl);
-    } else if (wave == 2) {
-      factor16<GT, FLV>(s.a, Bn, pub, Wn, lane, s.Y + (size_t)(k & 1) * FLV * 256, s.S + (k & 1) * 17, yl);
-    } else if (wave == 3 && k + 1 < nw) {
+    } else if (k + 1 < nw) {
       // G[w', w'], G[w', w], G[w, w'] of the next window w' from B[k % 2], which the updates of
       // window k - 1 write
       if (k > 0) {
-        long long polls = 0;
         bool ok = true;
+        long long polls = 0;
         while (__hip_atomic_load(applied + (k - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < done) {
           if (++polls > s.a.wait_limit) { ok = false; break; }
           __builtin_amdgcn_s_sleep(1);
@@ -1394,6 +1442,7 @@ __device__ __forceinline__ void slice16_role(const WindowSlice<GT>& s, unsigned 
           v[2][b][q] = Gb[(size_t)rp + (size_t)cw * n];
         }
       }
+      wait_count(&pub->formed, FLV * k);         // window k's block has read its operands
 #pragma unroll
       for (int b = 0; b < FLV; b++)
 #pragma unroll
@@ -1401,14 +1450,7 @@ __device__ __forceinline__ void slice16_role(const WindowSlice<GT>& s, unsigned 
 #pragma unroll
           for (int mat = 0; mat < 3; mat++)
             pf[(3 * b + mat) * MAT + ((lane >> 4) + 4 * q) * LD + r] = v[mat][b][q];
-    }
-    __syncthreads();
-  }
-  if (wave == 2) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    if (lane == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      __hip_atomic_store(ready + (nw - 1), epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      set_count(&pub->fetched, k + 1, lane);
     }
   }
   if (tid == 0) {
@@ -1509,7 +1551,7 @@ __device__ __forceinline__ void apply_load_r(GT (&rv)[W / 4], const GT* Gb, int 
   }
 }
 
-template <typename GT, int W, typename Ready>
+template <typename GT, int W, bool SHARED, typename Ready>
 __device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __restrict__ Gs, const int* Sp,
                                            const GT* Y, int n, int wp, TileRun t, unsigned char* smem, Ready ready) {
   typedef typename V4<GT>::type acc_t;
@@ -1574,7 +1616,7 @@ __device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __res
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           GT* base = Gw + r0 + (size_t)(c0 + 16 * j + mfma_row<GT>(0, r)) * n;
-          *reinterpret_cast<GT*>(reinterpret_cast<char*>(base) + o) = cur.acc[j][r];
+          put<SHARED>(reinterpret_cast<GT*>(reinterpret_cast<char*>(base) + o), (GT)cur.acc[j][r]);
         }
     } else {
       const int grow = r0 + 16 * wave + li;
@@ -1583,7 +1625,7 @@ __device__ __forceinline__ void apply_tiles(GT* __restrict__ Gd, const GT* __res
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           const int gcol = c0 + 16 * j + mfma_row<GT>(lane, r);
-          if (grow < n && gcol < n) Gw[(size_t)grow + (size_t)gcol * n] = cur.acc[j][r];
+          if (grow < n && gcol < n) put<SHARED>(Gw + (size_t)grow + (size_t)gcol * n, (GT)cur.acc[j][r]);
         }
     }
     if (i + 1 < t.count) cur = nxt;
@@ -1602,7 +1644,7 @@ __global__ __launch_bounds__(256) void window_kernel(WindowArgs<GT> a) {
     return;
   }
   const int t = (int)blockIdx.x - 1;
-  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(t, t + 1, a.n), smem, []() {});
+  apply_tiles<GT, W, false>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(t, t + 1, a.n), smem, []() {});
 }
 
 // The last window's application alone.
@@ -1610,7 +1652,7 @@ template <typename GT, int W>
 __global__ __launch_bounds__(256) void window_apply_kernel(WindowArgs<GT> a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int t = (int)blockIdx.x;
-  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(t, t + 1, a.n), smem, []() {});
+  apply_tiles<GT, W, false>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(t, t + 1, a.n), smem, []() {});
 }
 
 // Bounded wait until *p >= v (device scope); false when the bound is reached.
@@ -1707,16 +1749,13 @@ __global__ __launch_bounds__(256) void window_slice_kernel(WindowSlice<GT> s) {
   for (int j = 0; j < s.nw; j++) {
     if (j >= 1) wait_for(applied + (j - 1), done);
     if (run.count > 0)
-      apply_tiles<GT, W>(s.B[(j + 1) & 1], s.B[j & 1], s.S + (j & 1) * (W + 1), s.Y + (j & 1) * ysz, s.a.n,
+      apply_tiles<GT, W, true>(s.B[(j + 1) & 1], s.B[j & 1], s.S + (j & 1) * (W + 1), s.Y + (j & 1) * ysz, s.a.n,
                          j * W, run, smem, [&]() { wait_for(ready + j, e + 1); });
     else
       wait_for(ready + j, e + 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+    stores_done();
     __syncthreads();
-    if (tid == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      __hip_atomic_fetch_add(applied + j, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (tid == 0) __hip_atomic_fetch_add(applied + j, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -1725,14 +1764,16 @@ constexpr size_t apply_lds() {
   return sizeof(GT) * (size_t)W * 65;
 }
 
-// Sites per window (delay_depth selects 16, 32 or 64 explicitly).  Per-flip work and the
-// m x m solves grow with W, the per-window block formation and factor build with 1 / W.
-// Measured with one launch per slice: 16 is faster up to n = 256 (config B 71.5 against
-// 73.7 ms per sweep; the 64-chain config-D batch 323 against 313 sweeps/s), 32 beyond
-// (n = 576: 326 against 335 ms; n = 1024: 373 against 406 ms).
+// Sites per window (delay_depth selects 16, 32 or 64 explicitly).  16-site windows have the faster
+// decisions (a 16-lane row holds a matrix); 32-site ones update G half as often, which counts
+// where an application workgroup has several tiles.  The line lies at one tile each (a slice
+// launch has at most 128 application workgroups).  Sweeps with 16 and 32 sites: n = 400, two
+// flavours (98 tiles) 21.8 and 23.9 ms; n = 576, one flavour (81 tiles) 179 and 198 ms; n = 576, two
+// flavours (162 tiles) 43.1 and 40.9 ms; n = 784 (169) 60.3 and 56.4 ms; n = 1024, two flavours
+// (512) 212 and 196 ms.
 int window_size(int n, int flv) {
-  (void)flv;
-  return n <= 256 ? 16 : 32;
+  const int nt = (n + 63) / 64;
+  return flv * nt * nt <= 128 ? 16 : 32;
 }
 
 template <typename GT, int FLV, int W>
@@ -1775,7 +1816,7 @@ __global__ __launch_bounds__(256) void window_multi_kernel(const WindowArgs<GT>*
   const int nt = (a.n + 63) / 64;
   const int tile = (int)blockIdx.x - 1;
   if (tile >= a.flv * nt * nt) return;
-  apply_tiles<GT, W>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(tile, tile + 1, a.n), smem, []() {});
+  apply_tiles<GT, W, false>(a.Gd, a.G, a.Sp, a.Yp, a.n, a.wp, tile_run(tile, tile + 1, a.n), smem, []() {});
 }
 
 template <int W>
