@@ -41,24 +41,26 @@ __device__ __forceinline__ fx4 mfma16(float a, float b, fx4 c) {
 
 // Tile geometry: TILE x TILE outputs per workgroup, K staged in chunks of KC.  TILE = 32
 // (a wave: one 16x16 fragment) where a launch has few tiles, TILE = 64 (a wave: a 32x32 quadrant
-// as 2 x 2 fragments) where it has many: half the operand traffic per flop.  With either, an
-// element is the sum (p0 + p1) + (p2 + p3) of four accumulators, p_q over the pieces
-// k = 16 (4 i + q) .. + 15, i = 0, 1, ..., in order, so the two give identical results: a wave of
-// the 32-wide tile holds one of the four, a wave of the 64-wide tile two.
+// as 2 x 2 fragments; two workgroups per CU) where it has many: half the operand traffic per
+// flop.  With either, an element is the sum (p0 + p2) + (p1 + p3) of four accumulators, p_q over
+// the pieces k = 16 (4 i + q) .. + 15, i = 0, 1, ..., in order, so the two give identical
+// results: a wave of the 32-wide tile holds one of the four, a wave of the 64-wide tile p_g and
+// p_(g+2), whose sum it forms itself.
 template <int TILE> struct TileCfg {
   static constexpr int Threads = TILE == 32 ? 1024 : 512;
   static constexpr int Groups = Threads / 256;            // waves per quadrant
   static constexpr int Parts = 4 / Groups;                // accumulators per wave and fragment
-  static constexpr int KC = TILE == 32 ? 128 : 64;
+  static constexpr int KC = TILE == 32 ? 128 : 32;
   static constexpr int LD = TILE + 1;
   static constexpr int F = TILE / 32;                     // 16x16 fragments per wave and side
-  static constexpr int LPT = 2 * TILE * KC / Threads;     // loads per thread per chunk (8, 16)
+  static constexpr int LPT = 2 * TILE * KC / Threads;     // loads per thread per chunk (8)
+  static constexpr int Blocks = TILE == 32 ? 1 : 2;       // workgroups per CU
 };
 
 template <typename T, int TILE>
 constexpr size_t gemm_lds_bytes() {
   const size_t stage = sizeof(T) * 2 * 2 * TileCfg<TILE>::KC * TileCfg<TILE>::LD;
-  const size_t sums = sizeof(T) * 16 * TileCfg<TILE>::F * TileCfg<TILE>::F * 16 * 17;
+  const size_t sums = sizeof(T) * TileCfg<TILE>::Groups * 4 * TileCfg<TILE>::F * TileCfg<TILE>::F * 16 * 17;
   return stage > sums ? stage : sums;
 }
 
@@ -88,7 +90,7 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by, int& bz) {
 // the kernel arguments (a separate instantiation, so the one-chain path reads its items
 // straight from the argument segment)
 template <typename T, int TA, int TB, bool TAB, int TILE>
-__global__ __launch_bounds__(TileCfg<TILE>::Threads) void gemm_kernel(GemmBatch<T> batch) {
+__global__ __launch_bounds__(TileCfg<TILE>::Threads, TileCfg<TILE>::Threads * TileCfg<TILE>::Blocks / 256) void gemm_kernel(GemmBatch<T> batch) {
   typedef typename AccT<T>::type acc_t;
   constexpr int kTM = TILE, kTN = TILE, kKC = TileCfg<TILE>::KC, kLD = TileCfg<TILE>::LD;
   constexpr int kF = TileCfg<TILE>::F, kLoadsPerThread = TileCfg<TILE>::LPT;
@@ -217,29 +219,26 @@ __global__ __launch_bounds__(TileCfg<TILE>::Threads) void gemm_kernel(GemmBatch<
 #pragma unroll
       for (int j = 0; j < kF; j++) acc[h][i][j] = mfma16(av[i], bv[j], acc[h][i][j]);
   };
-  auto compute = [&](int c, int buf) {
-    const T* Ab = As + buf * kKC * kLD;
-    const T* Bb = Bs + buf * kKC * kLD;
-    const int kend = K - c * kKC < kKC ? K - c * kKC : kKC;
-    // (a whole chunk: straight-line k-steps, so the LDS reads run ahead of the products)
-    const bool whole = kend == kKC;
+  // 16 k-steps of a piece (offset k0 in a chunk with kend of K left): a whole one straight-line,
+  // so that the LDS reads run ahead of the products
+  auto piece = [&](const T* Ab, const T* Bb, int k0, int kend, int h) {
+    if (k0 + 16 <= kend) {
 #pragma unroll
-    for (int p = 0; p < kKC; p += 64)
+      for (int kk = 0; kk < 16; kk += 4) step(Ab, Bb, k0 + kk, h);
+    } else {
 #pragma unroll
-      for (int h = 0; h < kParts; h++) {
-        const int k0 = p + 16 * (kq + kGroups * h);
-        if (whole || k0 + 16 <= kend) {
-#pragma unroll
-          for (int kk = 0; kk < 16; kk += 4) step(Ab, Bb, k0 + kk, h);
-        } else {
-#pragma unroll
-          for (int kk = 0; kk < 16; kk += 4)
-            if (k0 + kk < kend) step(Ab, Bb, k0 + kk, h);
-        }
-      }
+      for (int kk = 0; kk < 16; kk += 4)
+        if (k0 + kk < kend) step(Ab, Bb, k0 + kk, h);
+    }
   };
 
   if constexpr (TILE == 32) {
+    auto compute = [&](int c, int buf) {
+      // (not unrolled over the pieces: the registers of 16 waves)
+#pragma unroll 1
+      for (int p = 0; p < kKC; p += 64)
+        piece(As + buf * kKC * kLD, Bs + buf * kKC * kLD, p + 16 * kq, K - c * kKC, 0);
+    };
     // chunk c lives in buffer c % 2 and arrives in register set ra (even c) or rb (odd c), so
     // that two chunks are in flight
     T ra[kLoadsPerThread], rb[kLoadsPerThread];
@@ -260,33 +259,40 @@ __global__ __launch_bounds__(TileCfg<TILE>::Threads) void gemm_kernel(GemmBatch<
       }
     }
   } else {
-    // one chunk ahead: its loads take no longer than a chunk's products
+    // a chunk holds two of the four pieces, in turn; one chunk ahead (the CU's other workgroup
+    // computes while this one waits)
     T ra[kLoadsPerThread];
     load(0, ra);
     store(0, ra);
     __syncthreads();
-    for (int c = 0; c < nch; c++) {
+    for (int c = 0; c < nch; c += 2) {
       if (c + 1 < nch) load(c + 1, ra);
-      compute(c, c & 1);
-      if (c + 1 < nch) store((c + 1) & 1, ra);
+      piece(As, Bs, 16 * kq, K - c * kKC, 0);
+      if (c + 1 < nch) store(1, ra);
       __syncthreads();
+      if (c + 1 < nch) {
+        if (c + 2 < nch) load(c + 2, ra);
+        piece(As + kKC * kLD, Bs + kKC * kLD, 16 * kq, K - (c + 1) * kKC, 1);
+        if (c + 2 < nch) store(0, ra);
+        __syncthreads();
+      }
     }
   }
 
-  // the four partial sums of every element through LDS (free after the last barrier): fragment
-  // (piece, quadrant, i, j) at 272 elements each, column by column with leading dimension 17
+  // the partial sums of every element through LDS (free after the last barrier): fragment
+  // (group, quadrant, i, j) at 272 elements each, column by column with leading dimension 17
   T* red = reinterpret_cast<T*>(smem);
-  constexpr int kFrag = 16 * 17, kQuarter = 4 * kF * kF * kFrag;
+  constexpr int kFrag = 16 * 17, kGroup = 4 * kF * kF * kFrag;
 #pragma unroll
-  for (int h = 0; h < kParts; h++)
+  for (int i = 0; i < kF; i++)
 #pragma unroll
-    for (int i = 0; i < kF; i++)
+    for (int j = 0; j < kF; j++)
 #pragma unroll
-      for (int j = 0; j < kF; j++)
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          red[(kq + kGroups * h) * kQuarter + ((quad * kF + i) * kF + j) * kFrag + li * 17 + mfma_row<T>(lane, r)] =
-              acc[h][i][j][r];
+      for (int r = 0; r < 4; r++) {
+        T x = acc[0][i][j][r];
+        if constexpr (kParts == 2) x += acc[1][i][j][r];
+        red[kq * kGroup + ((quad * kF + i) * kF + j) * kFrag + li * 17 + mfma_row<T>(lane, r)] = x;
+      }
   __syncthreads();
 
   const T alpha = T(batch.alpha), beta = T(batch.beta);
@@ -302,7 +308,10 @@ __global__ __launch_bounds__(TileCfg<TILE>::Threads) void gemm_kernel(GemmBatch<
     if (row >= M || col >= N) continue;
     const int qd = rt / (16 * kF) + 2 * (ct / (16 * kF)), i = rt / 16 % kF, j = ct / 16 % kF;
     const T* x = red + ((qd * kF + i) * kF + j) * kFrag + (ct & 15) * 17 + (rt & 15);
-    T v = alpha * ((x[0] + x[kQuarter]) + (x[2 * kQuarter] + x[3 * kQuarter]));
+    T sum;
+    if constexpr (kParts == 2) sum = x[0] + x[kGroup];
+    else sum = (x[0] + x[2 * kGroup]) + (x[kGroup] + x[3 * kGroup]);
+    T v = alpha * sum;
     if (has_l) v *= T(diag_at(it.dl, row));
     if (has_r) v *= T(diag_at(it.dr, col));
     T* dst = Cm + (size_t)row + (size_t)col * ldc;
@@ -312,14 +321,14 @@ __global__ __launch_bounds__(TileCfg<TILE>::Threads) void gemm_kernel(GemmBatch<
   }
 }
 
-// Which tile: one workgroup per CU at a time (LDS), so a launch lasts its rounds of 256 workgroups.
-// A round costs the tile's products (K / 4 steps of 64 clocks on every SIMD for TILE = 32, four
-// times that for 64) and its fill, sums and stores, about 6000 clocks (32) or 12000 (64).
+// Which tile: a launch lasts its rounds of one 32-wide or two 64-wide workgroups per CU.  A round
+// costs the products (K / 4 steps of 64 clocks on every SIMD per 32-wide tile, four times that per
+// 64-wide one) and the fill, sums and stores, about 6000 and 8000 clocks.
 constexpr int64_t kGemmCUs = 256;
 static bool wide_tiles(int64_t t32, int64_t t64, int K) {
   const int64_t step = (int64_t)((K + 3) / 4) * 64;
   const int64_t c32 = (t32 + kGemmCUs - 1) / kGemmCUs * (step + 6000);
-  const int64_t c64 = (t64 + kGemmCUs - 1) / kGemmCUs * (4 * step + 12000);
+  const int64_t c64 = (t64 + kGemmCUs - 1) / kGemmCUs * 4 * step + 8000;
   return c64 < c32;
 }
 
