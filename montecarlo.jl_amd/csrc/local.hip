@@ -6,14 +6,14 @@
 // of linalg/updates.jl:7-131.
 //
 // Design: the sites of a slice are visited in windows of W in {16, 32, 64} consecutive
-// sites, one launch per window:
+// sites, in one launch per slice (window_slice_kernel) or one per window:
 //  * workgroup 0 forms the window's W x W block of G (applying the previous window's
 //    factors to it), runs the Metropolis decisions and rank-1 updates on the block held in
 //    registers, and writes the dense factor Y of the accumulated update
 //    G <- G - C Y R with C = (I - G)[:, w], R = G[w, :] over the window's positions w;
 //  * workgroups 1.. apply the previous window's update to all of G on the matrix cores,
-//    one 64 x 64 tile each, from one copy of G into the other;
-//  * window_apply_kernel applies the last window's update.
+//    64 x 64 tiles, from one copy of G into the other;
+//  * one launch per window: window_apply_kernel applies the last window's update.
 // This is algebraically the reference's sequence of rank-1 updates; only the rounding
 // differs, so accept decisions agree except at ties |u - p| ~ 1e-12, which are counted.
 #include "common.h"
@@ -447,12 +447,8 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
       for (int c = 0; c < 16; c++) {
         const int cl = c < Wn ? c : Wn - 1;
         lo[c] = Bf[cl * LD + rc] * ((rok && c < Wn) ? 1.0 : 0.0);
-        if constexpr (W > 16) {
-          const int ch = c + 16 < Wn ? c + 16 : Wn - 1;
-          hi[c] = Bf[ch * LD + rc] * ((rok && c + 16 < Wn) ? 1.0 : 0.0);
-        } else {
-          hi[c] = 0.0;
-        }
+        const int ch = c + 16 < Wn ? c + 16 : Wn - 1;
+        hi[c] = Bf[ch * LD + rc] * ((rok && c + 16 < Wn) ? 1.0 : 0.0);
       }
       double dg = Bf[rc * LD + rc] * (rok ? 1.0 : 0.0);
       // the other flavour block's diagonal entry of this row, updated with the same
@@ -503,7 +499,7 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
         const double gam0t = readlane_f64(gq, t);
         const double gam1t = FLV > 1 ? readlane_f64(gq, 32 + t) : 0.0;
         const double gamL = f ? gam1t : gam0t;                    // this lane's block
-        const double gt = (W <= 16 || t < 16) ? lo[t & 15] : hi[t & 15];   // G_f[r][t]
+        const double gt = t < 16 ? lo[t & 15] : hi[t & 15];   // G_f[r][t]
         double* Vr = Vw + (size_t)(fb * W + m) * W;                        // raw row t
         const double uraw = (r == t ? 1.0 : 0.0) - gt;                     // u_t(r), unscaled
         if (fok && r < W) UwT[(size_t)(f * W + r) * UT + m] = uraw;         // u^T: [f][r][flip]
@@ -511,7 +507,7 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
 #pragma unroll
           for (int c = 0; c < 16; c += 2) {
             *reinterpret_cast<d2*>(Vr + c) = d2{lo[c], lo[c + 1]};
-            if constexpr (W > 16) *reinterpret_cast<d2*>(Vr + 16 + c) = d2{hi[c], hi[c + 1]};
+            *reinterpret_cast<d2*>(Vr + 16 + c) = d2{hi[c], hi[c + 1]};
           }
         }
         site_r = lane == m ? t : site_r;
@@ -531,11 +527,9 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
           const d2 vl = *reinterpret_cast<const d2*>(Vr + c);
           lo[c] = fma(-ug, vl[0], lo[c]);
           lo[c + 1] = fma(-ug, vl[1], lo[c + 1]);
-          if constexpr (W > 16) {
-            const d2 vh = *reinterpret_cast<const d2*>(Vr + 16 + c);
-            hi[c] = fma(-ug, vh[0], hi[c]);
-            hi[c + 1] = fma(-ug, vh[1], hi[c + 1]);
-          }
+          const d2 vh = *reinterpret_cast<const d2*>(Vr + 16 + c);
+          hi[c] = fma(-ug, vh[0], hi[c]);
+          hi[c + 1] = fma(-ug, vh[1], hi[c + 1]);
         }
         dg = fma(-ug, Vr[rw], dg);
         if constexpr (FLV > 1) {
@@ -1251,7 +1245,7 @@ __device__ __forceinline__ int factor16(const WindowArgs<GT>& a, const double* B
       }
       if (fin <= k) break;
     }
-    const int t = __builtin_amdgcn_readfirstlane(pub->site[k]);
+    const int t = __builtin_amdgcn_readfirstlane(pub->site[k]) & 15;   // (a case of the tables, always)
     const double gam = pub->gam[k][fb];
     double brt, prt, unused;                     // B[r][t], P[r][t]
     swap16(x[t], brt, unused);
