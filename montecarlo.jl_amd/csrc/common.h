@@ -144,7 +144,7 @@ struct RdivpBatch {
   const RdivpItem* items = nullptr;   // many-chain launches: device table, own n <= max_n
   int max_n = 0;
 };
-constexpr int kRdivpStripMaxN = 1024;  // one wave per 16-row strip up to this size
+constexpr int kRdivpStripMaxN = 1024;  // one workgroup per 16-row strip, the strip in LDS, up to this size
 hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s);
 
 // Elementwise helpers (util.hip)

@@ -902,148 +902,162 @@ __global__ __launch_bounds__(256) void rdivp_kernel(RdivpBatch batch) {
   }
 }
 
-// rdivp for n <= kRdivpStripMaxN: one wave per 16-row strip.  The strip's pivoted input
-// is gathered into LDS once (X[k][r], column-major per strip) and every solved column
-// stays there, so a panel's coupling X_{<J} T_{<J,J} reads only T from global memory.
-static size_t rdivp_strip_lds_bytes(int n) { return ((size_t)n * 17 + 2 * 16 * 17) * 8 + (size_t)n * 4; }
+// rdivp for kRdivpBlockMaxN < n <= kRdivpStripMaxN: five waves per 16-row strip, the form of
+// rdivp_block_kernel with the diagonal blocks' inverses made on the way (all of them at once
+// would not fit in LDS beside the strip).  Per 16-column panel p:
+//   waves 0 to 3 share Y = X_p - X_{<p} T_{<p,p} on the matrix cores (wave w takes k-steps w, w + 4,
+//   ...) and then issue the loads of T's coupling column of panel p + 1;
+//   wave 4 inverts the diagonal block of panel p + 1 (lane c solves U x = e_c upwards);
+//   wave 0 forms X_p = Y inv(T_pp), one 16 x 16 x 16 product.
+// What bounds a panel is the latency of T's column (16 lines per load, issued a panel's reduction
+// ahead) and the inversion beside it.  One wave per strip with a substitution per panel took 269
+// us at n = 576 and 709 us at n = 1024 (two matrices); this takes 199 and 560 us.
+// KS = 40 (n <= 640) or 64: k-steps of one wave per panel, at most.  Sums run in the order of
+// rdivp_block_kernel, so an item's result does not depend on the launch it shares.
+static size_t rdivp_wide_lds_bytes(int n) {
+  return ((size_t)n * 17 + 3 * 16 * 17 + 4 * 4 * 64 + 16 * 17) * 8 + (size_t)n * 4;
+}
 
-template <bool TAB>
-__global__ __launch_bounds__(64) void rdivp_strip_kernel(RdivpBatch batch) {
-  constexpr bool tab = TAB;
-  const RdivpItem it = tab ? batch.items[blockIdx.y] : batch.it[blockIdx.y];
-  const int n = tab ? it.n : batch.n;
-  const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
+template <bool TAB, int KS>
+__global__ __launch_bounds__(320) void rdivp_wide_kernel(RdivpBatch batch) {
+  const RdivpItem it = TAB ? batch.items[blockIdx.y] : batch.it[blockIdx.y];
+  const int n = TAB ? it.n : batch.n;
   const int r0 = blockIdx.x * 16;
   if (TAB && r0 >= n) return;   // item-table launches size the grid for the largest item
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = (n + 15) / 16;
   extern __shared__ __align__(16) unsigned char smem[];
-  double* X = reinterpret_cast<double*>(smem);   // [n][17]
-  double* Ysh = X + (size_t)n * 17;              // [16][17]
-  double* Tsh = Ysh + 16 * 17;                   // [16][17]
-  int* pv = reinterpret_cast<int*>(Tsh + 16 * 17);
+  double* X = reinterpret_cast<double*>(smem);          // [n][17]: X[j * 17 + row]
+  double* Ti = X + (size_t)n * 17;                      // [2][16][17]: inverses of even and odd panels
+  double* Ub = Ti + 2 * 16 * 17;                        // [16][17]: the block wave 4 inverts
+  double* red = Ub + 16 * 17;                           // [4 waves][4][64]
+  double* Ysh = red + 4 * 4 * 64;                       // [16][17]: Y[row][col]
+  int* pv = reinterpret_cast<int*>(Ysh + 16 * 17);
   double* __restrict__ A = it.A;
   const double* __restrict__ T = it.T;
-  const int rr = r0 + li;
-  const int rc = rr < n ? rr : n - 1;
 
-  for (int j0 = 0; j0 < n; j0 += 64 * 16) {
-    int t[16];
+  for (int j = tid; j < n; j += 320) pv[j] = it.pivot[j];
+  __syncthreads();
+  // the strip's pivoted input (thread: row tid % 16, columns tid / 16 + 20 q)
+  const int grow = tid & 15, gcol = tid >> 4;
+  const int grr = r0 + grow, grc = grr < n ? grr : n - 1;
+  for (int jb = 0; jb < n; jb += 320) {
+    double v[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int j = j0 + lane + 64 * q;
-      t[q] = it.pivot[j < n ? j : n - 1];
+      const int j = jb + gcol + 20 * q;
+      v[q] = A[(size_t)grc + (size_t)pv[j < n ? j : n - 1] * n];
     }
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int j = j0 + lane + 64 * q;
-      if (j < n) pv[j] = t[q];
+      const int j = jb + gcol + 20 * q;
+      if (j < n) X[(size_t)j * 17 + grow] = v[q];
     }
   }
-  __syncthreads();
-  // O[r][j] = A[r][pivot[j]]: lane (row li, phase lk) takes columns lk + 4 q
-  for (int jb = 0; jb < n; jb += 128) {
-    double v[32];
-#pragma unroll
-    for (int q = 0; q < 32; q++) {
-      const int j = jb + lk + 4 * q;
-      v[q] = A[(size_t)rc + (size_t)pv[j < n ? j : n - 1] * n];
-    }
-#pragma unroll
-    for (int q = 0; q < 32; q++) {
-      const int j = jb + lk + 4 * q;
-      if (j < n) X[(size_t)j * 17 + li] = v[q];
-    }
-  }
-  __syncthreads();
-
-  // T of the next panel (its diagonal block and coupling rows k < 256) is loaded while the
-  // current panel is solved
-  constexpr int kPre = 64;                       // prefetched coupling rows k = 4 q + lk
-  double td[4], tb[kPre];
-  auto load_t = [&](int j0n) {
-    const int cbn = j0n + li;
-    const int cbcn = cbn < n ? cbn : n - 1;
+  // wave 4: the diagonal block of panel p (lane: rows lk + 4 q of column li), the identity beyond n
+  double ub[4];
+  auto load_block = [&](int p) {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const int a = lk + 4 * q;
-      const int ta = j0n + a < n ? j0n + a : n - 1;
-      const double x = T[(size_t)ta + (size_t)cbcn * n];
-      td[q] = (j0n + a < n && cbn < n) ? x : (a == li ? 1.0 : 0.0);   // out of range: identity
-    }
-#pragma unroll
-    for (int g = 0; g < kPre / 16; g++) {
-      if (64 * g < j0n) {                        // uniform: 16 loads at once
-#pragma unroll
-        for (int q = 16 * g; q < 16 * g + 16; q++) {
-          const int k = 4 * q + lk;
-          tb[q] = T[(size_t)(k < j0n ? k : 0) + (size_t)cbcn * n];
-        }
-      }
+      const int ra = 16 * p + lk + 4 * q, cc = 16 * p + li;
+      const double v = T[(size_t)(ra < n ? ra : n - 1) + (size_t)(cc < n ? cc : n - 1) * n];
+      ub[q] = ra < n && cc < n ? (lk + 4 * q <= li ? v : 0.0) : (lk + 4 * q == li ? 1.0 : 0.0);
     }
   };
-  load_t(0);
-  for (int j0 = 0; j0 < n; j0 += 16) {
-    const int w = n - j0 < 16 ? n - j0 : 16;
-    const int cb = j0 + li;
-    const int cbc = cb < n ? cb : n - 1;
-    dx4 acc = dx4{0, 0, 0, 0};
+  auto invert = [&](int p) {
 #pragma unroll
-    for (int q = 0; q < kPre; q++)
-      if (4 * q < j0) acc = mfma16(X[(size_t)(4 * q + lk) * 17 + li], tb[q], acc);
-    for (int kb = 4 * kPre; kb < j0; kb += 128) {
-      double tc[32];
+    for (int q = 0; q < 4; q++) Ub[(lk + 4 * q) * 17 + li] = ub[q];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double x[16];
+    // x[k] = 0 for k > c, so every row runs the same straight-line sum
 #pragma unroll
-      for (int q = 0; q < 32; q++) {
-        const int k = kb + 4 * q + lk;
-        tc[q] = T[(size_t)(k < j0 ? k : 0) + (size_t)cbc * n];
-      }
+    for (int i = 15; i >= 0; i--) {
+      double sum = i == li ? 1.0 : 0.0;
 #pragma unroll
-      for (int q = 0; q < 32; q++) {
-        const int k = kb + 4 * q + lk;
-        if (kb + 4 * q < j0) acc = mfma16(X[(size_t)k * 17 + li], tc[q], acc);
-      }
+      for (int k = i + 1; k < 16; k++) sum -= Ub[i * 17 + k] * x[k];
+      x[i] = i <= li ? sum / Ub[i * 17 + i] : 0.0;
     }
-#pragma unroll
-    for (int q = 0; q < 4; q++) Tsh[(lk + 4 * q) * 17 + li] = td[q];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = mfma_row<double>(lane, r);
-      Ysh[row * 17 + li] = cb < n ? X[(size_t)cb * 17 + row] - acc[r] : 0.0;
-    }
-    if (j0 + 16 < n) load_t(j0 + 16);
-    __syncthreads();
+    double* Tp = Ti + (size_t)(p & 1) * 16 * 17;
     if (lane < 16) {
-      // right-looking: x_c = v_c / T_cc, then v_c' -= x_c T_cc' for every later c'.  The
-      // quotient comes from the reciprocal y = 1 / T_cc with one correction,
-      // x = q + (v - T_cc q) y, q = v y, which is the correctly rounded v / T_cc (Markstein)
-      // for the unit-modulus diagonal of a UDT's T; any other diagonal value divides.
-      const double dl = Tsh[lane * 17 + lane];
-      const double yl = 1.0 / dl;
-      double v[16], x[16];
 #pragma unroll
-      for (int c = 0; c < 16; c++) v[c] = Ysh[lane * 17 + c];
+      for (int a = 0; a < 16; a++) Tp[a * 17 + li] = x[a];
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  // waves 0 to 3: T's coupling column of panel j0 for this wave's k-steps q = wave + 4 s (4 q < j0)
+  double tb[KS];
+  auto load_tb = [&](int j0) {
+    const int cb = j0 + li, cbc = cb < n ? cb : n - 1;
 #pragma unroll
-      for (int c = 0; c < 16; c++) {
-        const double d = readlane_d(dl, c);
-        const double y = readlane_d(yl, c);
-        double xc;
-        if (fabs(d) >= 0.5 && fabs(d) <= 2.0) {
-          const double q0 = v[c] * y;
-          xc = fma(fma(-d, q0, v[c]), y, q0);
-        } else {
-          xc = v[c] / d;
+    for (int g = 0; g < KS / 8; g++)
+      if (128 * g < j0) {
+#pragma unroll
+        for (int s = 8 * g; s < 8 * g + 8; s++) {
+          const int k = 4 * (wave + 4 * s) + lk;
+          tb[s] = T[(size_t)(k < j0 ? k : 0) + (size_t)cbc * n];
         }
-        x[c] = xc;
-#pragma unroll
-        for (int c2 = c + 1; c2 < 16; c2++) v[c2] -= xc * Tsh[c * 17 + c2];
       }
+  };
+  if (wave == 4) {
+    load_block(0);
+    invert(0);
+    if (nb > 1) load_block(1);
+  } else if (nb > 1) {
+    load_tb(16);
+  }
+  __syncthreads();
+  for (int p = 0; p < nb; p++) {
+    const int j0 = 16 * p;
+    if (wave < 4) {
+      dx4 acc = dx4{0, 0, 0, 0};
 #pragma unroll
-      for (int c = 0; c < 16; c++)
-        if (c < w) X[(size_t)(j0 + c) * 17 + lane] = x[c];
+      for (int g = 0; g < KS / 8; g++)
+        if (128 * g < j0) {
+#pragma unroll
+          for (int s = 8 * g; s < 8 * g + 8; s++) {
+            const int q = wave + 4 * s;
+            if (4 * q < j0) acc = mfma16(X[(size_t)(4 * q + lk) * 17 + li], tb[s], acc);
+          }
+        }
+#pragma unroll
+      for (int r = 0; r < 4; r++) red[(wave * 4 + r) * 64 + lane] = acc[r];
+      if (p >= 1 && p + 1 < nb) load_tb(j0 + 16);
+    } else if (p + 1 < nb) {
+      invert(p + 1);
+      if (p + 2 < nb) load_block(p + 2);
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int cb = j0 + li;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int row = mfma_row<double>(lane, r);
+        const double u = (red[r * 64 + lane] + red[(4 + r) * 64 + lane]) +
+                         (red[(8 + r) * 64 + lane] + red[(12 + r) * 64 + lane]);
+        Ysh[row * 17 + li] = cb < n ? X[(size_t)cb * 17 + row] - u : 0.0;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const double* Tp = Ti + (size_t)(p & 1) * 16 * 17;
+      dx4 o = dx4{0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) {
+        const int k = 4 * ks + lk;
+        o = mfma16(Ysh[li * 17 + k], Tp[k * 17 + li], o);
+      }
+      if (cb < n) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) X[(size_t)cb * 17 + mfma_row<double>(lane, r)] = o[r];
+      }
     }
     __syncthreads();
   }
-  if (rr < n) {
-    for (int j = lk; j < n; j += 4) A[(size_t)rr + (size_t)j * n] = X[(size_t)j * 17 + li];
+  if (grr < n) {
+    for (int j = gcol; j < n; j += 20) A[(size_t)grr + (size_t)j * n] = X[(size_t)j * 17 + grow];
   }
 }
 
@@ -1205,9 +1219,12 @@ hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s) {
     else if (b.max_n <= kRdivpBlockMaxN)
       hipLaunchKernelGGL((rdivp_block_kernel<true, 32>), dim3((b.max_n + 15) / 16, b.count), dim3(256),
                          rdivp_block_lds_bytes(b.max_n), s, b);
+    else if (b.max_n <= 640)
+      hipLaunchKernelGGL((rdivp_wide_kernel<true, 40>), dim3((b.max_n + 15) / 16, b.count), dim3(320),
+                         rdivp_wide_lds_bytes(b.max_n), s, b);
     else if (b.max_n <= kRdivpStripMaxN)
-      hipLaunchKernelGGL(rdivp_strip_kernel<true>, dim3((b.max_n + 15) / 16, b.count), dim3(64),
-                         rdivp_strip_lds_bytes(b.max_n), s, b);
+      hipLaunchKernelGGL((rdivp_wide_kernel<true, 64>), dim3((b.max_n + 15) / 16, b.count), dim3(320),
+                         rdivp_wide_lds_bytes(b.max_n), s, b);
     else
       hipLaunchKernelGGL(rdivp_kernel<true>, dim3((b.max_n + 63) / 64, b.count), dim3(256), 0, s, b);
     return hipGetLastError();
@@ -1219,9 +1236,12 @@ hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s) {
   else if (b.n <= kRdivpBlockMaxN)
     hipLaunchKernelGGL((rdivp_block_kernel<false, 32>), dim3((b.n + 15) / 16, b.count), dim3(256),
                        rdivp_block_lds_bytes(b.n), s, b);
+  else if (b.n <= 640)
+    hipLaunchKernelGGL((rdivp_wide_kernel<false, 40>), dim3((b.n + 15) / 16, b.count), dim3(320),
+                       rdivp_wide_lds_bytes(b.n), s, b);
   else if (b.n <= kRdivpStripMaxN)
-    hipLaunchKernelGGL(rdivp_strip_kernel<false>, dim3((b.n + 15) / 16, b.count), dim3(64),
-                       rdivp_strip_lds_bytes(b.n), s, b);
+    hipLaunchKernelGGL((rdivp_wide_kernel<false, 64>), dim3((b.n + 15) / 16, b.count), dim3(320),
+                       rdivp_wide_lds_bytes(b.n), s, b);
   else
     hipLaunchKernelGGL(rdivp_kernel<false>, dim3((b.n + 63) / 64, b.count), dim3(256), 0, s, b);
   return hipGetLastError();
@@ -1236,8 +1256,10 @@ hipError_t qr_kernels_init() {
                        reinterpret_cast<const void*>(udt_panel_tall_kernel<false>),
                        reinterpret_cast<const void*>(udt_panel_tall_kernel<true>),
                        reinterpret_cast<const void*>(udt_panel_tab_kernel),
-                       reinterpret_cast<const void*>(rdivp_strip_kernel<false>),
-                       reinterpret_cast<const void*>(rdivp_strip_kernel<true>),
+                       reinterpret_cast<const void*>(rdivp_wide_kernel<false, 40>),
+                       reinterpret_cast<const void*>(rdivp_wide_kernel<true, 40>),
+                       reinterpret_cast<const void*>(rdivp_wide_kernel<false, 64>),
+                       reinterpret_cast<const void*>(rdivp_wide_kernel<true, 64>),
                        reinterpret_cast<const void*>(rdivp_block_kernel<false, 16>),
                        reinterpret_cast<const void*>(rdivp_block_kernel<true, 16>),
                        reinterpret_cast<const void*>(rdivp_block_kernel<false, 32>),
