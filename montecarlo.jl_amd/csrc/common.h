@@ -119,15 +119,13 @@ hipError_t launch_udt_norms(const UdtBatch& b, hipStream_t s);
 hipError_t launch_udt_panel(const UdtBatch& b, int p0, int w, int last, hipStream_t s);
 hipError_t launch_udt_reflect(const UdtBatch& b, int p0, int w, hipStream_t s);
 hipError_t launch_udt_finish(const UdtBatch& b, hipStream_t s);
-// Item-table forms (b.items set): every item's panel (p0, w, last) is in its table entry;
-// the panel kernel's rows-per-thread class R (1, 2, 4, 8: rows <= 256 R) is the same for all
-// items of one launch.  max_w bounds the items' panel widths.
+// Item-table forms (b.items set): every item's panel (p0, w, last) is in its table entry; the
+// panel kernel's class R (1: 16 columns, up to 1024 rows; 8: 8 columns beyond) is the same for
+// all items of one launch.
 int udt_rows_class(int rows);
 int udt_width_for(int rows);
 hipError_t launch_udt_panel_tab(const UdtBatch& b, int R, hipStream_t s);
 hipError_t launch_udt_reflect_tab(const UdtBatch& b, int max_grid, hipStream_t s);
-// Q accumulation into U (U preset to I) for every panel, in one launch
-
 
 // rdivp: A <- A[:, pivot] * triu(T)^-1 with O as n*n scratch (qr.hip).
 struct RdivpItem {
