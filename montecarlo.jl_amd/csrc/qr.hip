@@ -195,7 +195,8 @@ __device__ __forceinline__ double wave_total(double v) {
 // nu = copysign(||x||, x1), xi = x1 + nu and g = 1 / (nu xi) from normu = ||x||^2 > 0, so that
 // H a = a - u (u^T a) g with u = (xi, x_2, x_3, ...).  Inside a range where nothing can overflow
 // or turn subnormal the root comes from the hardware estimate by Goldschmidt's iteration and the
-// reciprocal by Newton's (each refined past double precision); outside, the library forms.
+// reciprocal by Newton's (each to the last bits of a double); outside, where nu xi need not have a
+// finite reciprocal, g = -xi / nu = -tau, and H a = a - v tau (v^T a) with v = u / xi.
 __device__ __forceinline__ void reflector_scalars(double normu, double x1, double& nu, double& xi, double& g) {
   if (normu >= 0x1p-900 && normu <= 0x1p900) {
     const double y = __builtin_amdgcn_rsq(normu);
@@ -215,7 +216,7 @@ __device__ __forceinline__ void reflector_scalars(double normu, double x1, doubl
   } else {
     nu = copysign(sqrt(normu), x1);
     xi = x1 + nu;
-    g = 1.0 / (nu * xi);
+    g = -(xi / nu);
   }
 }
 
@@ -289,7 +290,8 @@ __device__ __forceinline__ void panel_choice(const UdtItem& it, int n, int p0, i
 // instructions per wave and the waves' work runs beside each other.  Column j, once final, is
 // published in LDS (x below its diagonal, zero elsewhere); every later column's wave forms its
 // x^T a while column j's wave forms ||x||^2 and the scalars, and then applies
-//   a <- a - u (u^T a) g,  u = (xi, x), g = 1 / (nu xi)   (reflector_scalars).
+//   a <- a - u (u^T a) g,  u = (xi, x), g = 1 / (nu xi)   (reflector_scalars, with its form for
+// squared norms next to the ends of the range).
 // A column's wave depends only on lower columns' waves of the same workgroup, in order, so the
 // waits end; the chain is 16 steps of one reduction, one root and one reciprocal.
 // What bounds it is that chain's latency, and beside it the issue slots of the 16 waves on four
@@ -376,11 +378,16 @@ __device__ __forceinline__ void panel_body(const UdtItem& it, int n, int p0, int
       while (__hip_atomic_load(pub + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= j) {}
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
       const double xj = scal[2 * j], g = scal[2 * j + 1];
-      if (g != 0.0) {                            // 0: a zero column, H = I
+      if (g > 0.0) {
         const double f = fma(aj, xj, tot) * g;
         a[0] = fma(-(lane == j ? xj : x[0]), f, a[0]);
 #pragma unroll
         for (int k = 1; k < RT; k++) a[k] = fma(-x[k], f, a[k]);
+      } else if (g != 0.0) {                     // -tau (or NaN); 0: a zero column, H = I
+        const double r = 1.0 / xj, f = -g * fma(tot, r, aj);
+        a[0] = fma(-(lane == j ? 1.0 : x[0] * r), f, a[0]);
+#pragma unroll
+        for (int k = 1; k < RT; k++) a[k] = fma(-(x[k] * r), f, a[k]);
       }
     }
     // column c is final: x below the diagonal, then the scalars
