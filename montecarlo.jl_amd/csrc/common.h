@@ -142,7 +142,11 @@ struct RdivpBatch {
   const RdivpItem* items = nullptr;   // many-chain launches: device table, own n <= max_n
   int max_n = 0;
 };
-constexpr int kRdivpStripMaxN = 1024;  // one workgroup per 16-row strip, the strip in LDS, up to this size
+// The kernels' sizes: inverses of T's diagonal blocks up to kRdivpBlockMaxN, substitution with the
+// strip in LDS up to kRdivpStripMaxN, substitution in global memory beyond.  Items of one launch
+// lie in one of the three, so that an item's result does not depend on the launch it shares.
+constexpr int kRdivpBlockMaxN = 512;
+constexpr int kRdivpStripMaxN = 1024;
 hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s);
 
 // Elementwise helpers (util.hip)

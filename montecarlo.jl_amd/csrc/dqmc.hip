@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -1697,7 +1698,7 @@ int executor_step(Executor* x, Chain* const* cs, int nc) {
   }
   std::vector<GemmItem<double>> gt;
   std::vector<UdtItem> ut;
-  std::vector<RdivpItem> rt, rt2;
+  std::vector<RdivpItem> rt;
   std::vector<ElemItem> et;
   std::vector<MaxdiffItem> mt;
   for (auto& kv : groups) {
@@ -1732,18 +1733,22 @@ int executor_step(Executor* x, Chain* const* cs, int nc) {
           break;
         }
         case kOpRdivp: {
-          rt.clear(); rt2.clear();
-          int m1 = 0, m2 = 0;
-          for (int i : mem) {
-            const RecOp& o = cs[i]->ops[q];
-            for (int k = 0; k < o.count; k++) {
-              const RdivpItem& r = cs[i]->rrdivp[o.first + k];
-              if (r.n <= kRdivpStripMaxN) { rt.push_back(r); m1 = std::max(m1, r.n); }
-              else { rt2.push_back(r); m2 = std::max(m2, r.n); }
+          // one launch per kernel class (common.h)
+          const int lim[] = {0, kRdivpBlockMaxN, kRdivpStripMaxN, INT_MAX};
+          for (int c = 0; c < 3; c++) {
+            rt.clear();
+            int mx = 0;
+            for (int i : mem) {
+              const RecOp& o = cs[i]->ops[q];
+              for (int k = 0; k < o.count; k++) {
+                const RdivpItem& r = cs[i]->rrdivp[o.first + k];
+                if (r.n <= lim[c] || r.n > lim[c + 1]) continue;
+                rt.push_back(r);
+                mx = std::max(mx, r.n);
+              }
             }
+            if (!rt.empty()) x->launches.push_back({6, x->put(rt.data(), rt.size()), (int)rt.size(), mx, 0, 0, 0, 0, 0, 0});
           }
-          if (!rt.empty()) x->launches.push_back({6, x->put(rt.data(), rt.size()), (int)rt.size(), m1, 0, 0, 0, 0, 0, 0});
-          if (!rt2.empty()) x->launches.push_back({6, x->put(rt2.data(), rt2.size()), (int)rt2.size(), m2, 0, 0, 0, 0, 0, 0});
           break;
         }
         case kOpElem: {

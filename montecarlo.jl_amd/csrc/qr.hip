@@ -909,24 +909,26 @@ __global__ __launch_bounds__(256) void rdivp_kernel(RdivpBatch batch) {
   }
 }
 
-// rdivp for kRdivpBlockMaxN < n <= kRdivpStripMaxN: five waves per 16-row strip, the form of
-// rdivp_block_kernel with the diagonal blocks' inverses made on the way (all of them at once
-// would not fit in LDS beside the strip).  Per 16-column panel p:
-//   waves 0 to 3 share Y = X_p - X_{<p} T_{<p,p} on the matrix cores (wave w takes k-steps w, w + 4,
+// rdivp for kRdivpBlockMaxN < n <= kRdivpStripMaxN: four waves per 16-row strip, the strip in LDS.
+// Per 16-column panel p:
+//   the waves share Y = X_p - X_{<p} T_{<p,p} on the matrix cores (wave w takes k-steps w, w + 4,
 //   ...) and then issue the loads of T's coupling column of panel p + 1;
-//   wave 4 inverts the diagonal block of panel p + 1 (lane c solves U x = e_c upwards);
-//   wave 0 forms X_p = Y inv(T_pp), one 16 x 16 x 16 product.
-// What bounds a panel is the latency of T's column (16 lines per load, issued a panel's reduction
-// ahead) and the inversion beside it.  One wave per strip with a substitution per panel took 269
-// us at n = 576 and 709 us at n = 1024 (two matrices); this takes 199 and 560 us.
-// KS = 40 (n <= 640) or 64: k-steps of one wave per panel, at most.  Sums run in the order of
-// rdivp_block_kernel, so an item's result does not depend on the launch it shares.
+//   wave 0 solves X_p T_pp = Y by substitution, row l % 16 in lane l (the quarters of the wave alike),
+//   T_pp's entries read from LDS at one address for all lanes;
+//   wave 1 brings T's diagonal block of panel p + 1 and its reciprocals to LDS beside it.
+// What bounds a panel is the substitution's chain and the latency of T's column (16 lines per load,
+// issued a solve ahead).  One matrix, n = 576 and 1024: one wave per strip 279 and 751 us; five waves,
+// one of which inverts the next diagonal block for a product in place of the substitution, 204 and
+// 568 us; this, four waves with all their registers (no spills), 170 and 439 us.  The product's residual
+// also grows with the inverse's entries (a unit-diagonal block with entries of size 3: from 3e-16 to
+// 1e-9 of |X| |T|), and its 0 times infinity spoils columns that do not depend on an infinite entry.
+// KS = 40 (n <= 640) or 64: k-steps of one wave per panel, at most.
 static size_t rdivp_wide_lds_bytes(int n) {
-  return ((size_t)n * 17 + 3 * 16 * 17 + 4 * 4 * 64 + 16 * 17) * 8 + (size_t)n * 4;
+  return ((size_t)n * 17 + 2 * 16 * 17 + 2 * 16 + 4 * 4 * 64 + 16 * 17) * 8 + (size_t)n * 4;
 }
 
 template <bool TAB, int KS>
-__global__ __launch_bounds__(320) void rdivp_wide_kernel(RdivpBatch batch) {
+__global__ __launch_bounds__(256) void rdivp_wide_kernel(RdivpBatch batch) {
   const RdivpItem it = TAB ? batch.items[blockIdx.y] : batch.it[blockIdx.y];
   const int n = TAB ? it.n : batch.n;
   const int r0 = blockIdx.x * 16;
@@ -936,65 +938,53 @@ __global__ __launch_bounds__(320) void rdivp_wide_kernel(RdivpBatch batch) {
   const int nb = (n + 15) / 16;
   extern __shared__ __align__(16) unsigned char smem[];
   double* X = reinterpret_cast<double*>(smem);          // [n][17]: X[j * 17 + row]
-  double* Ti = X + (size_t)n * 17;                      // [2][16][17]: inverses of even and odd panels
-  double* Ub = Ti + 2 * 16 * 17;                        // [16][17]: the block wave 4 inverts
-  double* red = Ub + 16 * 17;                           // [4 waves][4][64]
+  double* Tsh = X + (size_t)n * 17;                     // [2][16][17]: diagonal blocks of even and odd panels
+  double* rec = Tsh + 2 * 16 * 17;                      // [2][16]: their diagonals' reciprocals
+  double* red = rec + 2 * 16;                           // [4 waves][4][64]
   double* Ysh = red + 4 * 4 * 64;                       // [16][17]: Y[row][col]
   int* pv = reinterpret_cast<int*>(Ysh + 16 * 17);
   double* __restrict__ A = it.A;
   const double* __restrict__ T = it.T;
 
-  for (int j = tid; j < n; j += 320) pv[j] = it.pivot[j];
+  for (int j = tid; j < n; j += 256) pv[j] = it.pivot[j];
   __syncthreads();
-  // the strip's pivoted input (thread: row tid % 16, columns tid / 16 + 20 q)
+  // the strip's pivoted input (thread: row tid % 16, columns tid / 16 + 16 q)
   const int grow = tid & 15, gcol = tid >> 4;
   const int grr = r0 + grow, grc = grr < n ? grr : n - 1;
-  for (int jb = 0; jb < n; jb += 320) {
+  for (int jb = 0; jb < n; jb += 256) {
     double v[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int j = jb + gcol + 20 * q;
+      const int j = jb + gcol + 16 * q;
       v[q] = A[(size_t)grc + (size_t)pv[j < n ? j : n - 1] * n];
     }
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int j = jb + gcol + 20 * q;
+      const int j = jb + gcol + 16 * q;
       if (j < n) X[(size_t)j * 17 + grow] = v[q];
     }
   }
-  // wave 4: the diagonal block of panel p (lane: rows lk + 4 q of column li), the identity beyond n
+  // wave 1: the diagonal block of panel p (lane: rows lk + 4 q of column li), the identity beyond n
   double ub[4];
   auto load_block = [&](int p) {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int ra = 16 * p + lk + 4 * q, cc = 16 * p + li;
       const double v = T[(size_t)(ra < n ? ra : n - 1) + (size_t)(cc < n ? cc : n - 1) * n];
-      ub[q] = ra < n && cc < n ? (lk + 4 * q <= li ? v : 0.0) : (lk + 4 * q == li ? 1.0 : 0.0);
+      ub[q] = ra < n && cc < n ? v : (lk + 4 * q == li ? 1.0 : 0.0);
     }
   };
-  auto invert = [&](int p) {
+  auto store_block = [&](int p) {
+    double* Tp = Tsh + (size_t)(p & 1) * 16 * 17;
+    double d = 1.0;
 #pragma unroll
-    for (int q = 0; q < 4; q++) Ub[(lk + 4 * q) * 17 + li] = ub[q];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    double x[16];
-    // x[k] = 0 for k > c, so every row runs the same straight-line sum
-#pragma unroll
-    for (int i = 15; i >= 0; i--) {
-      double sum = i == li ? 1.0 : 0.0;
-#pragma unroll
-      for (int k = i + 1; k < 16; k++) sum -= Ub[i * 17 + k] * x[k];
-      x[i] = i <= li ? sum / Ub[i * 17 + i] : 0.0;
+    for (int q = 0; q < 4; q++) {
+      Tp[(lk + 4 * q) * 17 + li] = ub[q];
+      d = lk + 4 * q == li ? ub[q] : d;
     }
-    double* Tp = Ti + (size_t)(p & 1) * 16 * 17;
-    if (lane < 16) {
-#pragma unroll
-      for (int a = 0; a < 16; a++) Tp[a * 17 + li] = x[a];
-    }
-    __builtin_amdgcn_wave_barrier();
+    if (lk == (li & 3)) rec[(p & 1) * 16 + li] = 1.0 / d;
   };
-  // waves 0 to 3: T's coupling column of panel j0 for this wave's k-steps q = wave + 4 s (4 q < j0)
+  // T's coupling column of panel j0 for this wave's k-steps q = wave + 4 s (4 q < j0)
   double tb[KS];
   auto load_tb = [&](int j0) {
     const int cb = j0 + li, cbc = cb < n ? cb : n - 1;
@@ -1008,34 +998,28 @@ __global__ __launch_bounds__(320) void rdivp_wide_kernel(RdivpBatch batch) {
         }
       }
   };
-  if (wave == 4) {
+  if (wave == 1) {
     load_block(0);
-    invert(0);
+    store_block(0);
     if (nb > 1) load_block(1);
-  } else if (nb > 1) {
-    load_tb(16);
   }
+  if (nb > 1) load_tb(16);
   __syncthreads();
   for (int p = 0; p < nb; p++) {
     const int j0 = 16 * p;
-    if (wave < 4) {
-      dx4 acc = dx4{0, 0, 0, 0};
+    dx4 acc = dx4{0, 0, 0, 0};
 #pragma unroll
-      for (int g = 0; g < KS / 8; g++)
-        if (128 * g < j0) {
+    for (int g = 0; g < KS / 8; g++)
+      if (128 * g < j0) {
 #pragma unroll
-          for (int s = 8 * g; s < 8 * g + 8; s++) {
-            const int q = wave + 4 * s;
-            if (4 * q < j0) acc = mfma16(X[(size_t)(4 * q + lk) * 17 + li], tb[s], acc);
-          }
+        for (int s = 8 * g; s < 8 * g + 8; s++) {
+          const int q = wave + 4 * s;
+          if (4 * q < j0) acc = mfma16(X[(size_t)(4 * q + lk) * 17 + li], tb[s], acc);
         }
+      }
 #pragma unroll
-      for (int r = 0; r < 4; r++) red[(wave * 4 + r) * 64 + lane] = acc[r];
-      if (p >= 1 && p + 1 < nb) load_tb(j0 + 16);
-    } else if (p + 1 < nb) {
-      invert(p + 1);
-      if (p + 2 < nb) load_block(p + 2);
-    }
+    for (int r = 0; r < 4; r++) red[(wave * 4 + r) * 64 + lane] = acc[r];
+    if (p >= 1 && p + 1 < nb) load_tb(j0 + 16);
     __syncthreads();
     if (wave == 0) {
       const int cb = j0 + li;
@@ -1049,22 +1033,43 @@ __global__ __launch_bounds__(320) void rdivp_wide_kernel(RdivpBatch batch) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const double* Tp = Ti + (size_t)(p & 1) * 16 * 17;
-      dx4 o = dx4{0, 0, 0, 0};
+      const double* Tp = Tsh + (size_t)(p & 1) * 16 * 17;
+      const double dl = Tp[li * 17 + li], yl = rec[(p & 1) * 16 + li];
+      double v[16];
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        const int k = 4 * ks + lk;
-        o = mfma16(Ysh[li * 17 + k], Tp[k * 17 + li], o);
-      }
-      if (cb < n) {
+      for (int c = 0; c < 16; c++) v[c] = Ysh[li * 17 + c];
+      // x_c = v_c / T_cc, then v_c' -= x_c T_cc' for every later c'.  The quotient comes from the
+      // reciprocal y = 1 / T_cc with one correction, x = q + (v - T_cc q) y, q = v y, which is the
+      // correctly rounded v / T_cc (Markstein) for the unit-modulus diagonal of a UDT's T (an infinite
+      // q stays); any other diagonal value divides.
 #pragma unroll
-        for (int r = 0; r < 4; r++) X[(size_t)cb * 17 + mfma_row<double>(lane, r)] = o[r];
+      for (int c = 0; c < 16; c++) {
+        const double d = readlane_d(dl, c), y = readlane_d(yl, c);
+        double xc;
+        if (fabs(d) >= 0.5 && fabs(d) <= 2.0) {
+          const double q0 = v[c] * y;
+          xc = fma(fma(-d, q0, v[c]), y, q0);
+          xc = fabs(q0) < HUGE_VAL ? xc : q0;
+        } else {
+          xc = v[c] / d;
+        }
+        v[c] = xc;
+#pragma unroll
+        for (int c2 = c + 1; c2 < 16; c2++) v[c2] = fma(-xc, Tp[c * 17 + c2], v[c2]);
       }
+      if (lane < 16) {
+#pragma unroll
+        for (int c = 0; c < 16; c++)
+          if (j0 + c < n) X[(size_t)(j0 + c) * 17 + lane] = v[c];
+      }
+    } else if (wave == 1 && p + 1 < nb) {
+      store_block(p + 1);
+      if (p + 2 < nb) load_block(p + 2);
     }
     __syncthreads();
   }
   if (grr < n) {
-    for (int j = gcol; j < n; j += 20) A[(size_t)grr + (size_t)j * n] = X[(size_t)j * 17 + grow];
+    for (int j = gcol; j < n; j += 16) A[(size_t)grr + (size_t)j * n] = X[(size_t)j * 17 + grow];
   }
 }
 
@@ -1076,8 +1081,6 @@ __global__ __launch_bounds__(320) void rdivp_wide_kernel(RdivpBatch batch) {
 // forms X_p = Y inv(T_pp), one 16 x 16 x 16 product.  In exact arithmetic this is the
 // column-by-column substitution of the reference; the products round differently (the
 // bound of the kernel tests: 1e-12 of the largest entry).
-constexpr int kRdivpBlockMaxN = 512;
-
 static size_t rdivp_block_lds_bytes(int n) {
   const size_t nb = (size_t)(n + 15) / 16;
   return ((size_t)n * 17 + nb * 16 * 17 + 4 * 4 * 64 + 16 * 17) * 8 + (size_t)n * 4;
@@ -1217,8 +1220,8 @@ __global__ __launch_bounds__(256) void rdivp_block_kernel(RdivpBatch batch) {
 hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s) {
   if (b.count <= 0) return hipSuccess;
   if (b.items) {
-    // item table: one kernel class per launch (the host keeps n <= kRdivpStripMaxN items
-    // and larger ones apart); the grid and LDS are sized for the largest item
+    // item table: one kernel class per launch (the host packs items of n <= kRdivpBlockMaxN, of
+    // n <= kRdivpStripMaxN and larger ones apart); the grid and LDS are sized for the largest item
     if (b.max_n < 1 || b.max_n > 2048) return hipErrorInvalidValue;
     if (b.max_n <= 256)
       hipLaunchKernelGGL((rdivp_block_kernel<true, 16>), dim3((b.max_n + 15) / 16, b.count), dim3(256),
@@ -1227,10 +1230,10 @@ hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s) {
       hipLaunchKernelGGL((rdivp_block_kernel<true, 32>), dim3((b.max_n + 15) / 16, b.count), dim3(256),
                          rdivp_block_lds_bytes(b.max_n), s, b);
     else if (b.max_n <= 640)
-      hipLaunchKernelGGL((rdivp_wide_kernel<true, 40>), dim3((b.max_n + 15) / 16, b.count), dim3(320),
+      hipLaunchKernelGGL((rdivp_wide_kernel<true, 40>), dim3((b.max_n + 15) / 16, b.count), dim3(256),
                          rdivp_wide_lds_bytes(b.max_n), s, b);
     else if (b.max_n <= kRdivpStripMaxN)
-      hipLaunchKernelGGL((rdivp_wide_kernel<true, 64>), dim3((b.max_n + 15) / 16, b.count), dim3(320),
+      hipLaunchKernelGGL((rdivp_wide_kernel<true, 64>), dim3((b.max_n + 15) / 16, b.count), dim3(256),
                          rdivp_wide_lds_bytes(b.max_n), s, b);
     else
       hipLaunchKernelGGL(rdivp_kernel<true>, dim3((b.max_n + 63) / 64, b.count), dim3(256), 0, s, b);
@@ -1244,10 +1247,10 @@ hipError_t launch_rdivp(const RdivpBatch& b, hipStream_t s) {
     hipLaunchKernelGGL((rdivp_block_kernel<false, 32>), dim3((b.n + 15) / 16, b.count), dim3(256),
                        rdivp_block_lds_bytes(b.n), s, b);
   else if (b.n <= 640)
-    hipLaunchKernelGGL((rdivp_wide_kernel<false, 40>), dim3((b.n + 15) / 16, b.count), dim3(320),
+    hipLaunchKernelGGL((rdivp_wide_kernel<false, 40>), dim3((b.n + 15) / 16, b.count), dim3(256),
                        rdivp_wide_lds_bytes(b.n), s, b);
   else if (b.n <= kRdivpStripMaxN)
-    hipLaunchKernelGGL((rdivp_wide_kernel<false, 64>), dim3((b.n + 15) / 16, b.count), dim3(320),
+    hipLaunchKernelGGL((rdivp_wide_kernel<false, 64>), dim3((b.n + 15) / 16, b.count), dim3(256),
                        rdivp_wide_lds_bytes(b.n), s, b);
   else
     hipLaunchKernelGGL(rdivp_kernel<false>, dim3((b.n + 63) / 64, b.count), dim3(256), 0, s, b);
