@@ -1011,7 +1011,9 @@ typedef double d16 __attribute__((ext_vector_type(16)));
 // block jumps to case t of a table of straight-line cases.  The matrices sit in fixed registers,
 // x in v[96:127] and y in v[64:95], so that the block names their parts and updates them in place
 // (a switch around single updates made the compiler copy all 16 entries twice per flip).  The
-// wait states before the jump cover a register written just before the block.
+// wait states before the jump cover a register written just before the block.  The jump multiplies t
+// by a case's size in bytes, which the assembler checks at the end of every case: another encoding
+// of an instruction would send the jump into the middle of one.
 #define DQMC_ROW1(a, b, c, d, t) "v_fmac_f64_dpp v[" #a ":" #b "], v[" #c ":" #d "], %[l] row_newbcast:" #t \
                                  " row_mask:0xf bank_mask:0xf\n\t"
 #define DQMC_ROW_X(t) \
@@ -1030,9 +1032,12 @@ typedef double d16 __attribute__((ext_vector_type(16)));
   DQMC_ROW1(94, 95, 126, 127, t)
 // jump to case t of the table that follows, `size` bytes per case
 #define DQMC_ROW_JUMP(size) \
-  "s_nop 1\n\ts_mul_i32 s42, %[t], " #size "\n\ts_getpc_b64 s[40:41]\n.Lrow_pc%=:\n\t" \
+  ".set .Lrow_size%=, " #size "\n\ts_nop 1\n\ts_mul_i32 s42, %[t], .Lrow_size%=\n\ts_getpc_b64 s[40:41]\n.Lrow_pc%=:\n\t" \
   "s_add_u32 s40, s40, s42\n\ts_addc_u32 s41, s41, 0\n\ts_add_u32 s40, s40, .Lrow_tab%=-.Lrow_pc%=\n\t" \
   "s_addc_u32 s41, s41, 0\n\ts_setpc_b64 s[40:41]\n.Lrow_tab%=:\n\t"
+// end of case t
+#define DQMC_ROW_END(t) \
+  "s_branch .Lrow_end%=\n\t.if (.-.Lrow_tab%=)!=(" #t "+1)*.Lrow_size%=\n\t.error \"size of a row case\"\n\t.endif\n\t"
 #define DQMC_CASES16(M) \
   M(0, 96, 97) M(1, 98, 99) M(2, 100, 101) M(3, 102, 103) M(4, 104, 105) M(5, 106, 107) M(6, 108, 109) M(7, 110, 111) \
   M(8, 112, 113) M(9, 114, 115) M(10, 116, 117) M(11, 118, 119) M(12, 120, 121) M(13, 122, 123) M(14, 124, 125) \
@@ -1043,7 +1048,7 @@ __device__ __forceinline__ void row_flip(d16& x, double gq, double v, double w, 
   double l;
 #define DQMC_FLIP(t, a, b)                                                                                  \
   "v_mov_b64_dpp %[g], %[gq] row_newbcast:" #t " row_mask:0xf bank_mask:0xf\n\tv_mul_f64 %[l], %[g], %[v]\n\t" \
-  DQMC_ROW_X(t) "v_fma_f64 v[" #a ":" #b "], %[g], %[w], v[" #a ":" #b "]\n\ts_branch .Lrow_end%=\n\t"
+  DQMC_ROW_X(t) "v_fma_f64 v[" #a ":" #b "], %[g], %[w], v[" #a ":" #b "]\n\t" DQMC_ROW_END(t)
   asm volatile(DQMC_ROW_JUMP(156) DQMC_CASES16(DQMC_FLIP) ".Lrow_end%=:"
                : "+{v[96:127]}"(x), [g] "=&v"(gam), [l] "=&v"(l)
                : [gq] "v"(gq), [v] "v"(v), [w] "v"(w), [t] "s"(t)
@@ -1052,7 +1057,7 @@ __device__ __forceinline__ void row_flip(d16& x, double gq, double v, double w, 
 }
 // y[c] += l x[c][lane t], c = 0 .. 15.
 __device__ __forceinline__ void row_add(d16& y, d16& x, double l, int t) {
-#define DQMC_ADD(t, a, b) DQMC_ROW_Y(t) "s_branch .Lrow_end%=\n\t"
+#define DQMC_ADD(t, a, b) DQMC_ROW_Y(t) DQMC_ROW_END(t)
   asm volatile(DQMC_ROW_JUMP(132) DQMC_CASES16(DQMC_ADD) ".Lrow_end%=:"
                : "+{v[64:95]}"(y), "+{v[96:127]}"(x)
                : [l] "v"(l), [t] "s"(t)
@@ -1061,7 +1066,7 @@ __device__ __forceinline__ void row_add(d16& y, d16& x, double l, int t) {
 }
 // x[c] += l x[c][lane t], c = 0 .. 15.
 __device__ __forceinline__ void row_update(d16& x, double l, int t) {
-#define DQMC_UPD(t, a, b) DQMC_ROW_X(t) "s_branch .Lrow_end%=\n\t"
+#define DQMC_UPD(t, a, b) DQMC_ROW_X(t) DQMC_ROW_END(t)
   asm volatile(DQMC_ROW_JUMP(132) DQMC_CASES16(DQMC_UPD) ".Lrow_end%=:"
                : "+{v[96:127]}"(x)
                : [l] "v"(l), [t] "s"(t)
@@ -1071,6 +1076,7 @@ __device__ __forceinline__ void row_update(d16& x, double l, int t) {
 #undef DQMC_ROW1
 #undef DQMC_ROW_X
 #undef DQMC_ROW_Y
+#undef DQMC_ROW_END
 #undef DQMC_ROW_JUMP
 #undef DQMC_CASES16
 
