@@ -1,7 +1,6 @@
-"""The slice launch's update of G when a workgroup owns several 64 x 64 tiles (more than 128
-tiles in all): runs of tiles that cross a column of tiles and the boundary between the flavour
-blocks, and a ragged last tile, give the chain of one launch per window (one tile per
-workgroup) bit for bit."""
+"""The slice launch's update of G when a workgroup owns one or several 64 x 64 tiles (several from
+129 tiles on), and a ragged last tile, gives the chain of one launch per window (one tile per
+workgroup) bit for bit.  Runs across the boundary of the flavour blocks: test_gpu_tile_runs.py."""
 import numpy as np
 import pytest
 
@@ -10,8 +9,8 @@ from conftest import make_chain
 pytestmark = pytest.mark.gpu
 
 
-# n = 576: 162 tiles in runs of 2 over columns of 9; n = 729 (ragged, one block of 144 tiles);
-# n = 784 (ragged, 338 tiles in runs of 3 over columns of 13)
+# (U > 0: one flavour)  n = 576: 81 tiles, one per workgroup; n = 729 (ragged), two flavours: 288
+# tiles in runs of 3 down columns of 12; n = 784 (ragged): 169 tiles in runs of 2 across columns of 13
 @pytest.mark.parametrize("L,U,W", [(24, 4.0, 32), (27, -4.0, 16), (28, 4.0, 0)])
 def test_runs_of_tiles_equal_single_tiles(pkg, hip, L, U, W):
     chains = []
