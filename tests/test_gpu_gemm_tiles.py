@@ -1,5 +1,6 @@
-"""The product on both tile geometries (64-wide from n = 1000 on for one matrix), at the edges of
-the tiles, of the K chunks (128 and 32) and of the 16-wide pieces of K."""
+"""The product at the edges of the tiles, of the K chunks (128 and 32) and of the 16-wide pieces of
+K: 32-wide tiles, and 64-wide ones at n = 1000 (one matrix takes them from n = 865 to 1024:
+test_gpu_gemm_wide_tiles.py)."""
 import numpy as np
 import pytest
 
