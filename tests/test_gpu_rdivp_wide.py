@@ -1,5 +1,5 @@
-"""rdivp with five waves per strip (513 to 1024 rows): around its limits and at ragged sizes, by
-the residual X triu(T) = A[:, piv], and equal to the four-wave form on the rows they share."""
+"""rdivp from 513 to 1024 rows: around its limits and at ragged sizes, by the residual
+X triu(T) = A[:, piv].  Large entries and infinities: test_gpu_rdivp_stability.py."""
 import numpy as np
 import pytest
 
