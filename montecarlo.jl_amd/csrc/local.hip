@@ -440,8 +440,6 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
       const double* Bf = Bn + (size_t)fb * W * LD;
       // every read in flight at once: in-range (clamped) addresses, masked by an exact
       // multiplication with 0 or 1 (the block is finite), no per-column branch
-      // every read in flight at once: in-range (clamped) addresses, masked by an exact
-      // multiplication with 0 or 1 (the block is finite), no per-column branch
       rowvec lo, hi;
 #pragma unroll
       for (int c = 0; c < 16; c++) {
@@ -502,7 +500,7 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
         const double gt = t < 16 ? lo[t & 15] : hi[t & 15];   // G_f[r][t]
         double* Vr = Vw + (size_t)(fb * W + m) * W;                        // raw row t
         const double uraw = (r == t ? 1.0 : 0.0) - gt;                     // u_t(r), unscaled
-        if (fok && r < W) UwT[(size_t)(f * W + r) * UT + m] = uraw;         // u^T: [f][r][flip]
+        if (fok) UwT[(size_t)(f * W + r) * UT + m] = uraw;                  // u^T: [f][r][flip]
         if (fok && r == t) {
 #pragma unroll
           for (int c = 0; c < 16; c += 2) {
@@ -515,12 +513,11 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
         __builtin_amdgcn_s_waitcnt(0xC07F);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (fok && r == m) gam[f * W + m] = gamL;
-        const int rw = r < W ? r : W - 1;
         const double ug = fok ? gamL * uraw : 0.0;
         double vo = 0.0, uo = 0.0;
         if constexpr (FLV > 1) {
-          vo = Vw[(size_t)(fo * W + m) * W + rw];                // G_{1-f}[t][r]
-          uo = UwT[(size_t)(fo * W + rw) * UT + m];             // u_t(r) of the other block
+          vo = Vw[(size_t)(fo * W + m) * W + r];                 // G_{1-f}[t][r]
+          uo = UwT[(size_t)(fo * W + r) * UT + m];              // u_t(r) of the other block
         }
 #pragma unroll
         for (int c = 0; c < 16; c += 2) {
@@ -531,7 +528,7 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
           hi[c] = fma(-ug, vh[0], hi[c]);
           hi[c + 1] = fma(-ug, vh[1], hi[c + 1]);
         }
-        dg = fma(-ug, Vr[rw], dg);
+        dg = fma(-ug, Vr[r], dg);
         if constexpr (FLV > 1) {
           const double ugo = (f ? gam0t : gam1t) * uo;           // the owner's ug, bit for bit
           dgo = fma(-ugo, vo, dgo);
@@ -813,7 +810,7 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
       double* Xs = Uw;                  // [b][j][c], leading dimension LD
       double* Bs = Vw;                  // [b][i][j] = Binv[j][i] (transposed), leading dimension LD
       const int f = lane >> 5, r = lane & 31;
-      if ((wave == 1 || wave == 2) && f < FLV && r < W) {
+      if ((wave == 1 || wave == 2) && f < FLV) {
         double* dst = (wave == 1 ? Xs : Bs) + (size_t)f * W * LD;
 #pragma unroll
         for (int j = 0; j < W; j++) dst[j * LD + r] = j < 16 ? fx_lo[j & 15] : fx_hi[j & 15];
@@ -858,7 +855,7 @@ __device__ __forceinline__ void window_role(const WindowArgs<GT>& a, unsigned ch
         const int b = mat >> 1;
         // unconditional in-range loads (sites[] is 0 beyond m), then the mask
         const double vl = Uw[(b * W + l) * LD + sites[j]];
-        const double vn = W <= 32 ? Vw[(b * W + j) * W + sites[l]] : Vw[(b * W + j) * LD + vpos<W>(sites[l])];
+        const double vn = Vw[(b * W + j) * LD + vpos<W>(sites[l])];
         const double gj = gam[b * W + j];
         const bool isl = (mat & 1) == 0;
         const bool keep = isl ? (l < j && j < m) : (j < l && l < m);
