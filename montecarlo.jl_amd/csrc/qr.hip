@@ -198,7 +198,7 @@ __device__ __forceinline__ double wave_total(double v) {
 // reciprocal by Newton's (each to the last bits of a double); outside, where nu xi need not have a
 // finite reciprocal, g = -xi / nu = -tau, and H a = a - v tau (v^T a) with v = u / xi.
 __device__ __forceinline__ void reflector_scalars(double normu, double x1, double& nu, double& xi, double& g) {
-  if (normu >= 0x1p-900 && normu <= 0x1p900) {
+  if (__builtin_expect(normu >= 0x1p-900 && normu <= 0x1p900, 1)) {
     const double y = __builtin_amdgcn_rsq(normu);
     double s = normu * y, h = 0.5 * y;
     const double r = fma(-s, h, 0.5);
@@ -291,7 +291,8 @@ __device__ __forceinline__ void panel_choice(const UdtItem& it, int n, int p0, i
 // published in LDS (x below its diagonal, zero elsewhere); every later column's wave forms its
 // x^T a while column j's wave forms ||x||^2 and the scalars, and then applies
 //   a <- a - u (u^T a) g,  u = (xi, x), g = 1 / (nu xi)   (reflector_scalars, with its form for
-// squared norms next to the ends of the range).
+// squared norms next to the ends of the range; marked unlikely, which keeps that form off the straight
+// path: 16x16 sites 51.2 -> 50.8 ms per sweep).
 // A column's wave depends only on lower columns' waves of the same workgroup, in order, so the
 // waits end; the chain is 16 steps of one reduction, one root and one reciprocal.
 // What bounds it is that chain's latency, and beside it the issue slots of the 16 waves on four
@@ -378,12 +379,12 @@ __device__ __forceinline__ void panel_body(const UdtItem& it, int n, int p0, int
       while (__hip_atomic_load(pub + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= j) {}
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
       const double xj = scal[2 * j], g = scal[2 * j + 1];
-      if (g > 0.0) {
+      if (__builtin_expect(g > 0.0, 1)) {
         const double f = fma(aj, xj, tot) * g;
         a[0] = fma(-(lane == j ? xj : x[0]), f, a[0]);
 #pragma unroll
         for (int k = 1; k < RT; k++) a[k] = fma(-x[k], f, a[k]);
-      } else if (g != 0.0) {                     // -tau (or NaN); 0: a zero column, H = I
+      } else if (__builtin_expect(g != 0.0, 0)) {   // -tau (or NaN); 0: a zero column, H = I
         const double r = 1.0 / xj, f = -g * fma(tot, r, aj);
         a[0] = fma(-(lane == j ? 1.0 : x[0] * r), f, a[0]);
 #pragma unroll
@@ -920,8 +921,9 @@ __global__ __launch_bounds__(256) void rdivp_kernel(RdivpBatch batch) {
 // issued a solve ahead).  One matrix, n = 576 and 1024: one wave per strip 279 and 751 us; five waves,
 // one of which inverts the next diagonal block for a product in place of the substitution, 204 and
 // 568 us; this, four waves with all their registers (no spills), 170 and 439 us.  The product's residual
-// also grows with the inverse's entries (a unit-diagonal block with entries of size 3: from 3e-16 to
-// 1e-9 of |X| |T|), and its 0 times infinity spoils columns that do not depend on an infinite entry.
+// also grows with the inverse's entries (one unit-diagonal block with normal entries of size 3: up to
+// 2e-13 of |X| |T|, the substitution's 2e-16), and its 0 times infinity spoils columns that do not depend
+// on an infinite entry.
 // KS = 40 (n <= 640) or 64: k-steps of one wave per panel, at most.
 static size_t rdivp_wide_lds_bytes(int n) {
   return ((size_t)n * 17 + 2 * 16 * 17 + 2 * 16 + 4 * 4 * 64 + 16 * 17) * 8 + (size_t)n * 4;
