@@ -13,7 +13,8 @@
 // tile has four (or two) waves, each with v_mfma_f64_16x16x4f64 (FP64) or
 // v_mfma_f32_16x16x4f32 (FP32) accumulators over their part of K, added through LDS at the end.
 // The waves of a SIMD share the loads and hide each other's latencies, where one wave per SIMD was
-// bound by its own instruction stream.  Operand layout of the 16x16x4 instructions (wave64, lane l):
+// bound by its own instruction stream.  (The 64-wide FP64 form has 128 registers per wave, two
+// workgroups per CU, and spills 8 to 21 of them.)  Operand layout of the 16x16x4 instructions (wave64, lane l):
 //   A (16 x 4): lane l supplies A[l % 16][l / 16]
 //   B (4 x 16): lane l supplies B[l / 16][l % 16]
 //   D (16 x 16): lane l holds D[row][l % 16], r = 0..3, with row = l / 16 + 4 r (FP64)
@@ -321,9 +322,17 @@ __global__ __launch_bounds__(TileCfg<TILE>::Threads, TileCfg<TILE>::Threads * Ti
   }
 }
 
-// Which tile: a launch lasts its rounds of one 32-wide or two 64-wide workgroups per CU.  A round
-// costs the products (K / 4 steps of 64 clocks on every SIMD per 32-wide tile, four times that per
-// 64-wide one) and the fill, sums and stores, about 6000 and 8000 clocks.
+// Which tile, by an estimate in clocks.  32-wide: workgroups of a CU follow each other, each with its
+// products (K / 4 steps of 64 clocks on every SIMD) and about 6000 clocks of fill, sums and stores.
+// 64-wide: a CU's workgroups run in pairs that share the matrix cores, so four times the products for
+// each of them, and 8000 clocks once, for the fill and stores that no neighbour hides.  That
+// counts a partly filled turn of 256 as a whole one, which is too much beside a neighbour: for one
+// matrix of n = 1025 to 1248, 1409 to 1536 and 1729 to 1824, 32-wide tiles are taken although 64-wide
+// ones are faster, by a quarter at most.
+// Measured, 32- and 64-wide, one matrix: n = 576 27 and 40 us, 784 54 and 56, 864 55 and 62, 865 70
+// and 62, 1024 80 and 70, 1100 115 and 105, 1300 162 and 121, 1800 435 and 330, 2048 565 and 362; sweeps
+// of 32 chains of n = 256, two flavours, 23.4 and 19.5 ms, of 256 chains of n = 64 22.0 and 18.4 ms,
+// of 256 chains of n = 16 15.8 and 18.3 ms (16.4 ms by the rule).
 constexpr int64_t kGemmCUs = 256;
 static bool wide_tiles(int64_t t32, int64_t t64, int K) {
   const int64_t step = (int64_t)((K + 3) / 4) * 64;

@@ -1767,7 +1767,10 @@ constexpr size_t apply_lds() {
 // launch has at most 128 application workgroups).  Sweeps with 16 and 32 sites: n = 400, two
 // flavours (98 tiles) 21.8 and 23.9 ms; n = 576, one flavour (81 tiles) 179 and 198 ms; n = 576, two
 // flavours (162 tiles) 43.1 and 40.9 ms; n = 784 (169) 60.3 and 56.4 ms; n = 1024, two flavours
-// (512) 212 and 196 ms.
+// (512) 212 and 196 ms.  With one launch per window, which has twice the launches and passes over G
+// with 16 sites, those stay the faster ones below the line, beta = 1: n = 400, two flavours 10.5 and
+// 12.5 ms, n = 676, one flavour (121 tiles) 18.6 and 20.9 ms; in mixed precision 10.1 and 11.8, 18.0
+// and 20.3 ms; 32 chains together 62.7 and 69.5, 131 and 136 ms.
 int window_size(int n, int flv) {
   const int nt = (n + 63) / 64;
   return flv * nt * nt <= 128 ? 16 : 32;
